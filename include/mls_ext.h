@@ -1,0 +1,34 @@
+/*
+ * mls_ext.h — entry points of libmls_hip.so for this package's own Python modules.
+ *
+ * They follow mls.h's conventions (host-side validation, status codes, the caller owns
+ * every buffer, work enqueued on `stream`) and carry no ABI version of their own: the
+ * modules and the library are built together.
+ */
+#ifndef MLS_EXT_H
+#define MLS_EXT_H
+
+#include "mls.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* ---------------------------------------------------------------- FP8 training */
+
+/* The fp8 operands of train/fp8.py:62-95 padded for the K-contiguous GEMM:
+ * out[r][c] = fp8(x[r][c] / scale[r]) as [rows][Cp], and, when out_t is not null, its
+ * transpose [cols][Rp], where Cp and Rp are cols and rows rounded up to 64 and every
+ * padding byte is 0 (a zero in both formats). e5m2: 1 for e5m2, 0 for e4m3. e4m3 NaN codes
+ * are written as zeros into a copy whose reduction axis is padded (cols % 64 != 0: out;
+ * rows % 64 != 0: out_t): mls_fp8_gemm decodes them to 0 at such a K
+ * (kernels/fp8_matmul.py:46). out, out_t: 16-byte aligned. */
+int mlsx_fp8_encode_pad(int e5m2, const void* x, int x_dt, int64_t rows, int64_t cols, int64_t ldx, float scale,
+                        const float* scale_ptr, int64_t scale_stride, uint8_t* out, uint8_t* out_t,
+                        mls_stream_t stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* MLS_EXT_H */

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 
 #include "../../include/mls.h"
+#include "../../include/mls_ext.h"
 
 namespace mls {
 

@@ -97,6 +97,11 @@ SIGNATURES = {
                                             _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _F, _P], _I),
 }
 
+# include/mls_ext.h: entry points of this package's own modules
+EXT_SIGNATURES = {
+    "mlsx_fp8_encode_pad": ([_I, _P, _I, _I64, _I64, _I64, _F, _P, _I64, _P, _P, _P], _I),
+}
+
 
 class HipKernelError(RuntimeError):
     """A HIP kernel entry point returned an error status."""
@@ -116,7 +121,7 @@ def load_library(path: str | os.PathLike | None = None) -> ctypes.CDLL:
             f"{p} is not built: run `python -c 'import __graft_entry__ as g; g.build()'` "
             "or `python mini-llm-stack_amd/csrc/build.py` (the HIP kernels have no fallback)")
     lib = ctypes.CDLL(str(p))
-    for name, (args, res) in SIGNATURES.items():
+    for name, (args, res) in (*SIGNATURES.items(), *EXT_SIGNATURES.items()):
         fn = getattr(lib, name)
         fn.argtypes, fn.restype = args, res
     if lib.mls_abi_version() != ABI_VERSION:

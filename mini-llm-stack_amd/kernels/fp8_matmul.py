@@ -155,6 +155,28 @@ def quantize_e4m3_t(x: torch.Tensor, scale) -> tuple[torch.Tensor, torch.Tensor]
     return _encode_t("quantize_e4m3_t", "mls_e4m3_encode_t", x, scale)
 
 
+def encode_padded(x: torch.Tensor, scale, *, e5m2: bool = False, transposed: bool = True):
+    """(bits, bits_t) of a 2-D device tensor x [R, C] for the fp8 GEMMs of FP8 training:
+    bits [R, Cp] and its transpose [C, Rp] (None unless `transposed`), with Cp and Rp the
+    sizes rounded up to 64 and zero bytes in the padding, so that a GEMM reducing over
+    either axis runs on the matrix cores whatever the token count. Same rounding as
+    quantize_e4m3 / quantize_e5m2; e4m3 NaN codes become zeros in a copy whose reduction axis
+    is padded, as fp8_matmul decodes them there. scale: a float or a 1-element tensor."""
+    fn = "encode_padded"
+    dev = require_hip(fn, x)
+    x2 = rows(x)
+    R, C = x2.shape
+    sa = _row_scale(scale, R, dev, fn, False)
+    if sa is None:
+        raise ValueError(f"{fn}: scale must be a float, a 1-element tensor or [M, 1]")
+    out = torch.empty(R, (C + 63) // 64 * 64, dtype=torch.uint8, device=dev)
+    out_t = torch.empty(C, (R + 63) // 64 * 64, dtype=torch.uint8, device=dev) if transposed else None
+    kernels.check(kernels.lib().mlsx_fp8_encode_pad(
+        int(e5m2), x2.data_ptr(), dt_code(x.dtype, fn), R, C, ld(x2), sa[0], sa[1], sa[2], out.data_ptr(),
+        None if out_t is None else out_t.data_ptr(), stream(dev)), fn)
+    return out, out_t
+
+
 def transpose_u8(t: torch.Tensor) -> torch.Tensor:
     """A contiguous [cols, rows] copy of a 2-D byte tensor (fp8 bits): the .t() of
     an fp8 operand, materialised for the K-contiguous GEMM."""
