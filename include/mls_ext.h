@@ -27,6 +27,16 @@ int mlsx_fp8_encode_pad(int e5m2, const void* x, int x_dt, int64_t rows, int64_t
                         const float* scale_ptr, int64_t scale_stride, uint8_t* out, uint8_t* out_t,
                         mls_stream_t stream);
 
+/* max |x| of n contiguous values in two steps (train/fp8.py:33-48, 86-87: the amax behind
+ * a per-tensor scale; NaN wins over every number, as in torch's amax). mlsx_absmax_parts
+ * writes MLSX_ABSMAX_PARTS partial maxima; mlsx_absmax_scales takes those of `tensors`
+ * tensors one after another and writes amax[t] and scale[t] = max(amax[t] / fp8_max, 1e-12)
+ * (one IEEE division; a NaN stays). */
+#define MLSX_ABSMAX_PARTS 1024
+int mlsx_absmax_parts(const void* x, int x_dt, int64_t n, float* parts, mls_stream_t stream);
+int mlsx_absmax_scales(const float* parts, int tensors, float fp8_max, float* amax, float* scale,
+                       mls_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

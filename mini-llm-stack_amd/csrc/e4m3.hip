@@ -285,6 +285,58 @@ __global__ __launch_bounds__(256) void fp8_encode_pad_kernel(const T* __restrict
   *reinterpret_cast<uint4*>(out_t + dr * rp + r0 + lc) = *reinterpret_cast<const uint4*>(t);
 }
 
+// max |x| over a grid-stride range, one partial per block: the fp32 patterns with the sign
+// cleared compare as unsigned integers in the order of the magnitudes, and a NaN's lies
+// above infinity's, so it wins as it does in torch's amax. HBM-bound, one read of x and no
+// temporary: a 180 MB fp32 weight 117 us as abs() and amax() -> 33 us.
+template <typename T>
+__global__ __launch_bounds__(256) void absmax_parts_kernel(const T* __restrict__ x, int64_t n, bool vec,
+                                                           uint32_t* __restrict__ parts) {
+  constexpr int V = 16 / sizeof(T);
+  const int64_t stride = (int64_t)gridDim.x * 256, tid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t nv = vec ? n / V : 0;
+  uint32_t m = 0;
+  auto take = [&](const uint4& u) __attribute__((always_inline)) {
+    const T* e = reinterpret_cast<const T*>(&u);
+#pragma unroll
+    for (int k = 0; k < V; ++k) m = max(m, __float_as_uint(to_f32(e[k])) & 0x7FFFFFFFu);
+  };
+  const uint4* xv = reinterpret_cast<const uint4*>(x);
+  int64_t i = tid;
+  for (; i + 3 * stride < nv; i += 4 * stride) {  // four loads in flight
+    const uint4 a = xv[i], b = xv[i + stride], c = xv[i + 2 * stride], d = xv[i + 3 * stride];
+    take(a); take(b); take(c); take(d);
+  }
+  for (; i < nv; i += stride) take(xv[i]);
+  for (int64_t j = nv * V + tid; j < n; j += stride) m = max(m, __float_as_uint(to_f32(x[j])) & 0x7FFFFFFFu);
+  __shared__ uint32_t red[4];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) parts[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+// One block per tensor over its MLSX_ABSMAX_PARTS partial maxima.
+__global__ __launch_bounds__(256) void absmax_scales_kernel(const uint32_t* __restrict__ parts, float fp8_max,
+                                                            float* __restrict__ amax, float* __restrict__ scale) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < MLSX_ABSMAX_PARTS / 256; ++i)
+    m = max(m, parts[(int64_t)blockIdx.x * MLSX_ABSMAX_PARTS + i * 256 + threadIdx.x]);
+  __shared__ uint32_t red[4];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const float a = __uint_as_float(max(max(red[0], red[1]), max(red[2], red[3])));
+    const float q = a / fp8_max;
+    if (amax) amax[blockIdx.x] = a;
+    if (scale) scale[blockIdx.x] = q < 1e-12f ? 1e-12f : q;
+  }
+}
+
 static int grid_for(int64_t work, int block) {
   int64_t g = cdiv(work, block);
   if (g > 65536) g = 65536;
@@ -452,4 +504,33 @@ extern "C" int mlsx_fp8_encode_pad(int e5m2, const void* x, int x_dt, int64_t ro
   if (!aligned(out, 16) || !aligned(out_t, 16)) return fail(MLS_ERR_ARG, "%s: outputs must be 16-byte aligned", fn);
   return e5m2 ? fp8_encode_pad<true>(fn, x, x_dt, rows, cols, ldx, scale, scale_ptr, scale_stride, out, out_t, stream)
               : fp8_encode_pad<false>(fn, x, x_dt, rows, cols, ldx, scale, scale_ptr, scale_stride, out, out_t, stream);
+}
+
+extern "C" int mlsx_absmax_parts(const void* x, int x_dt, int64_t n, float* parts, mls_stream_t stream) {
+  const char* fn = "mlsx_absmax_parts";
+  if (n < 1) return fail(MLS_ERR_ARG, "%s: n=%lld < 1", fn, (long long)n);
+  if (!x || !parts) return fail(MLS_ERR_ARG, "%s: null pointer", fn);
+  if (!is_float_dt(x_dt)) return fail(MLS_ERR_ARG, "%s: bad x dtype %d", fn, x_dt);
+  const bool vec = aligned(x, 16);
+  const dim3 grid(MLSX_ABSMAX_PARTS);
+  hipStream_t st = (hipStream_t)stream;
+  uint32_t* p = reinterpret_cast<uint32_t*>(parts);
+  if (x_dt == MLS_F32)
+    hipLaunchKernelGGL(absmax_parts_kernel<float>, grid, dim3(256), 0, st, (const float*)x, n, vec, p);
+  else if (x_dt == MLS_F16)
+    hipLaunchKernelGGL(absmax_parts_kernel<_Float16>, grid, dim3(256), 0, st, (const _Float16*)x, n, vec, p);
+  else
+    hipLaunchKernelGGL(absmax_parts_kernel<__bf16>, grid, dim3(256), 0, st, (const __bf16*)x, n, vec, p);
+  return check_launch(fn);
+}
+
+extern "C" int mlsx_absmax_scales(const float* parts, int tensors, float fp8_max, float* amax, float* scale,
+                                  mls_stream_t stream) {
+  const char* fn = "mlsx_absmax_scales";
+  if (tensors < 1 || tensors > 65535) return fail(MLS_ERR_ARG, "%s: %d tensors", fn, tensors);
+  if (!parts || (!amax && !scale)) return fail(MLS_ERR_ARG, "%s: null pointer", fn);
+  if (!(fp8_max > 0.0f)) return fail(MLS_ERR_ARG, "%s: fp8_max must be positive", fn);
+  hipLaunchKernelGGL(absmax_scales_kernel, dim3((unsigned)tensors), dim3(256), 0, (hipStream_t)stream,
+                     reinterpret_cast<const uint32_t*>(parts), fp8_max, amax, scale);
+  return check_launch(fn);
 }

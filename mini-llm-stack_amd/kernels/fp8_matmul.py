@@ -38,6 +38,7 @@ from kernels._hip import dt_code, ld, require_hip, rows, stream
 E4M3_MAX = 448.0
 E5M2_MAX = 57344.0
 _FORMATS = {"e4m3": 0, "e5m2": kernels.MLS_FP8_A_E5M2}
+_AMAX_DT = {torch.float32: kernels.MLS_F32, torch.float16: kernels.MLS_F16, torch.bfloat16: kernels.MLS_BF16}
 
 
 def decode_e4m3(bits: torch.Tensor) -> torch.Tensor:
@@ -175,6 +176,25 @@ def encode_padded(x: torch.Tensor, scale, *, e5m2: bool = False, transposed: boo
         int(e5m2), x2.data_ptr(), dt_code(x.dtype, fn), R, C, ld(x2), sa[0], sa[1], sa[2], out.data_ptr(),
         None if out_t is None else out_t.data_ptr(), stream(dev)), fn)
     return out, out_t
+
+
+def amax_scales(tensors, fp8_max: float) -> torch.Tensor | None:
+    """fp32 [2, len(tensors)] on the device: max |t| of every tensor and the per-tensor scale
+    max(amax / fp8_max, 1e-12), from one read of each; None where a tensor is not a dense
+    non-empty device tensor of a supported dtype (the caller's torch ops then apply)."""
+    dev = tensors[0].device
+    for t in tensors:
+        if t.device.type != "cuda" or t.device != dev or t.dtype not in _AMAX_DT or not t.is_contiguous() or t.numel() == 0:
+            return None
+    n, L, st = len(tensors), kernels.lib(), stream(dev)
+    parts = torch.empty(n, kernels.ABSMAX_PARTS, dtype=torch.float32, device=dev)
+    out = torch.empty(2, n, dtype=torch.float32, device=dev)
+    for i, t in enumerate(tensors):
+        kernels.check(L.mlsx_absmax_parts(t.data_ptr(), _AMAX_DT[t.dtype], t.numel(),
+                                          parts.data_ptr() + 4 * i * kernels.ABSMAX_PARTS, st), "amax_scales")
+    kernels.check(L.mlsx_absmax_scales(parts.data_ptr(), n, float(fp8_max), out.data_ptr(), out.data_ptr() + 4 * n, st),
+                  "amax_scales")
+    return out
 
 
 def transpose_u8(t: torch.Tensor) -> torch.Tensor:

@@ -20,7 +20,7 @@ from collections import deque
 import torch
 import torch.nn as nn
 
-from kernels.fp8_matmul import (E4M3_MAX, E5M2_MAX, dequantize_e4m3, encode_padded, fp8_matmul,
+from kernels.fp8_matmul import (E4M3_MAX, E5M2_MAX, amax_scales, dequantize_e4m3, encode_padded, fp8_matmul,
                                 quantize_e4m3, quantize_e5m2)
 
 
@@ -37,7 +37,10 @@ class DynamicScaler:
     def scale_for(self, t: torch.Tensor) -> float:
         if not self.enabled:
             return 1.0
-        amax = float(t.detach().abs().amax())
+        return self.scale_from_amax(float(t.detach().abs().amax()))
+
+    def scale_from_amax(self, amax: float) -> float:
+        """scale_for a tensor whose max |value| is known."""
         if not self.hist:  # nothing recorded yet: seed the window with this tensor
             self.hist.append(max(amax, 1e-12))
         s = max(self.hist) / self.fp8_max
@@ -87,7 +90,9 @@ class _FP8LinearFn(torch.autograd.Function):
         sx, sw = ctx.scales
         if ctx.use_kernel and dy.device.type == "cuda":
             xbt, wbt = ctx.saved_tensors
-            sdy = _grad_scale(dy, ctx.scale_grads)
+            # the just-in-time scale stays on the device (no host sync in the backward)
+            on_device = amax_scales([dy.detach()], E5M2_MAX) if ctx.scale_grads else None
+            sdy = on_device[1] if on_device is not None else _grad_scale(dy, ctx.scale_grads)
             # the e5m2 gradient in both layouts from one pass (dy for dx, dy^T for dw)
             dyb, dybt = encode_padded(dy, sdy, e5m2=True)
             dx = fp8_matmul(dyb, wbt, sdy, sw, torch.float32, a_format="e5m2")
@@ -113,10 +118,19 @@ class FP8Linear(nn.Module):
     def forward(self, x):
         shape = x.shape
         flat = x.reshape(-1, shape[-1])
-        y = _FP8LinearFn.apply(flat, self.weight, self.sx.scale_for(flat),
-                               self.sw.scale_for(self.weight), self.use_kernel,
-                               self.sx.enabled)
+        sx, sw = self._scales(flat)
+        y = _FP8LinearFn.apply(flat, self.weight, sx, sw, self.use_kernel, self.sx.enabled)
         return y.reshape(*shape[:-1], -1)
+
+    def _scales(self, flat):
+        """(activation scale, weight scale): with the kernels, both maxima come from one read
+        of each tensor and one copy to the host."""
+        if self.use_kernel and type(self.sx) is type(self.sw) is DynamicScaler and self.sx.enabled and self.sw.enabled:
+            got = amax_scales([flat.detach(), self.weight.detach()], E4M3_MAX)
+            if got is not None:
+                ax, aw = got[0].tolist()
+                return self.sx.scale_from_amax(ax), self.sw.scale_from_amax(aw)
+        return self.sx.scale_for(flat), self.sw.scale_for(self.weight)
 
 
 def convert_linears_to_fp8(model: nn.Module, enabled: bool = True,

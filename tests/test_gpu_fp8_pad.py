@@ -1,11 +1,13 @@
-"""The padded fp8 encoders behind FP8Linear's steps."""
+"""The padded fp8 encoders and the amax kernel behind FP8Linear's steps."""
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
-from kernels.fp8_matmul import encode_padded, fp8_matmul, quantize_e4m3, quantize_e5m2
+from kernels.fp8_matmul import (E4M3_MAX, E5M2_MAX, amax_scales, encode_padded, fp8_matmul, quantize_e4m3,
+                                quantize_e5m2)
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +46,27 @@ def test_padded_gemm_matches_ragged(dev, M, N, K):
     va, vb = (q.view(torch.float8_e4m3fn).double() for q in (qa, qb))
     bound = K * 2.0 ** -24 * 0.01 * (va.abs() @ vb.abs().t())
     assert float(((got - want).double().abs() - bound).max()) <= 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,off", [(1, 0), (7, 1), (4096, 0), (1_000_003, 0), (5_000_001, 3)])
+def test_amax_scales(dev, n, off, dtype):
+    """Bit-identical to torch's amax and to a host division rounded to fp32, aligned or not."""
+    x = torch.randn(n + off, generator=torch.Generator().manual_seed(n)).to(dtype).to(dev)[off:]
+    x[n // 2] = -9.5
+    y = torch.zeros(33, device=dev)  # an all-zero tensor takes the floor
+    amax, scale = amax_scales([x, y], E4M3_MAX).cpu()
+    want = float(x.abs().amax())
+    assert float(amax[0]) == want and float(amax[1]) == 0.0
+    assert float(scale[0]) == np.float32(want / E4M3_MAX) and float(scale[1]) == np.float32(1e-12)
+    for bad in (float("inf"), float("nan")):
+        x[0] = bad
+        got = amax_scales([x], E5M2_MAX).cpu()
+        assert np.array_equal(got.numpy().ravel(), np.float32([bad, bad]), equal_nan=True)
+
+
+def test_amax_scales_declines(dev):
+    """A layout or dtype that the kernel does not read is left to torch's own ops."""
+    x = torch.randn(8, 8, device=dev)
+    assert amax_scales([x.t()], 1.0) is None and amax_scales([x[:0]], 1.0) is None
+    assert amax_scales([x.double()], 1.0) is None and amax_scales([x.cpu()], 1.0) is None
