@@ -14,6 +14,20 @@
 extern "C" {
 #endif
 
+/* ---------------------------------------------------------------- weight-only GEMMs */
+
+/* mls_int8_gemm_ws / mls_int4_gemm_ws with a workspace of mlsx_wq_workspace bytes (256-byte
+ * aligned; 0: none): shapes whose tiles would not fill the GPU, or whose K is a multiple of
+ * 32 but not of 64, run with the reduction axis split over blocks and fp32 partial products
+ * in the workspace (gemm_ksplit.hip); every other call is the _ws one. */
+int64_t mlsx_wq_workspace(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group);
+int mlsx_int8_gemm(const void* a, int a_dt, int64_t lda, const int8_t* w, int64_t ldw, const void* s, int s_dt,
+                   void* c, int c_dt, int64_t ldc, int64_t M, int64_t N, int64_t K, void* workspace,
+                   int64_t ws_bytes, mls_stream_t stream);
+int mlsx_int4_gemm(const void* a, int a_dt, int64_t lda, const uint8_t* w, int64_t ldw, const void* s, int s_dt,
+                   int64_t ld_sn, int64_t ld_sg, int group, void* c, int c_dt, int64_t ldc, int64_t M, int64_t N,
+                   int64_t K, void* workspace, int64_t ws_bytes, mls_stream_t stream);
+
 /* ---------------------------------------------------------------- FP8 training */
 
 /* The fp8 operands of train/fp8.py:62-95 padded for the K-contiguous GEMM:

@@ -466,26 +466,27 @@ double small_cost(int64_t M, int64_t N, int64_t K, int wbits, int tm, int tn) {
 
 // Whether the 8-wavefront kernel's x slices of a TM-row-tile block fit in LDS (as
 // launch_small_wv sizes them), i.e. whether a tile height keeps x out of the registers.
-bool small_xls_fits(const SmallArgs& a, int wbits, bool s64, int tm, int tn, int ssz) {
+bool small_xls_fits(int64_t K, int G, int wbits, bool s64, int tm, int tn, int ssz) {
   const int ks = wbits == 4 && !s64 ? 128 : 64;
-  const int nsteps = a.K / ks;
+  const int nsteps = (int)(K / ks);
   if (nsteps < 16) return false;  // 4 wavefronts, no slices
   int steps = 1;
   while (steps < (nsteps + 7) / 8) steps *= 2;
-  const int sc = wbits == 4 ? 16 * tn * a.G * ssz + 64 * 8 * 4 : 0;
+  const int sc = wbits == 4 ? 16 * tn * G * ssz + 64 * 8 * 4 : 0;
   return (sc + 255) / 256 * 256 + 8 * 16 * tm * (steps * ks * 2 / 16) * 16 <= 160 * 1024;
 }
 
-template <int WBITS, typename AT, typename ST, bool S64 = false, bool SPLIT = false>
-int dispatch_small(SmallArgs a, hipStream_t st) {
-  static const int force = env_int("MLS_SMALL_TILE", 0);  // TM * 10 + TN (sweeps)
-  int best_tm = SPLIT ? 2 : 1, best_tn = 1;
+// The tile (row tiles x column tiles of 16) for a shape; the byte model's time.
+double pick_small_tile(int64_t M, int64_t N, int64_t K, int G, int wbits, bool s64, bool split, int ssz, int& best_tm,
+                       int& best_tn) {
+  best_tm = split ? 2 : 1;
+  best_tn = 1;
   double best = 1e300;
-  for (int tm = SPLIT ? 2 : 1; tm <= 4; tm *= 2)
+  for (int tm = split ? 2 : 1; tm <= 4; tm *= 2)
     for (int tn = 1; tn <= 4; tn *= 2) {
-      if (tm > (SPLIT ? 2 : 1) && a.M <= 16 * tm / 2) continue;  // a row tile mostly past M
-      if (WBITS == 4 && tm * tn > 8) continue;      // INT4 4 x 4 would spill registers
-      const double c = small_cost(a.M, a.N, a.K, WBITS, tm, tn);
+      if (tm > (split ? 2 : 1) && M <= 16 * tm / 2) continue;  // a row tile mostly past M
+      if (wbits == 4 && tm * tn > 8) continue;      // INT4 4 x 4 would spill registers
+      const double c = small_cost(M, N, K, wbits, tm, tn);
       // the model counts bytes only; the widening of every weight, once per block, costs
       // VALU time on top. A taller tile within 30% of the best byte count is taken when its
       // x slices fit in LDS: each weight is then widened for twice the rows (the reference's
@@ -493,13 +494,21 @@ int dispatch_small(SmallArgs a, hipStream_t st) {
       // g128 7.51 -> 6.91 us, g64 8.50 -> 7.33 us; across M = 32..256 x (2048^2, 4096^2,
       // 11008 x 4096) no shape measured slower than the bytes-only choice)
       const bool taller_tie = c <= best * 1.3 && tm > best_tm &&
-                              small_xls_fits(a, WBITS, S64, tm, tn, (int)sizeof(ST));
+                              small_xls_fits(K, G, wbits, s64, tm, tn, ssz);
       if (c < best * 0.999 || taller_tie) {
         best = c;
         best_tm = tm;
         best_tn = tn;
       }
     }
+  return best;
+}
+
+template <int WBITS, typename AT, typename ST, bool S64 = false, bool SPLIT = false>
+int dispatch_small(SmallArgs a, hipStream_t st) {
+  static const int force = env_int("MLS_SMALL_TILE", 0);  // TM * 10 + TN (sweeps)
+  int best_tm, best_tn;
+  pick_small_tile(a.M, a.N, a.K, a.G, WBITS, S64, SPLIT, (int)sizeof(ST), best_tm, best_tn);
   if (force && (!SPLIT || force / 10 >= 2)) {
     best_tm = force / 10;
     best_tn = force % 10;
@@ -574,6 +583,24 @@ static int small_impl(int wbits, const WqArgs& p, int64_t m_out) {
                                                    : dispatch_small<8, __bf16, float>(a, p.stream);
   return p.s_dt == MLS_F16 ? dispatch_small<8, _Float16, _Float16>(a, p.stream)
                            : dispatch_small<8, _Float16, float>(a, p.stream);
+}
+
+// us of this kernel for M rows (split rows: of the split matrix), fitted to 169 shapes (M = 17
+// .. 512 rows, 512 x 512 to 4096 x 11008; log error 6 to 22% rms): the byte model's MB a CU,
+// the MFMA tiles a block multiplies, the rounds of blocks. With x slices in LDS (8
+// wavefronts) the bytes cost a quarter of what per-lane loads do.
+float small_estimate_us(int wbits, int64_t M, int64_t N, int64_t K, int group, int ssz, bool split) {
+  const bool s64 = wbits == 4 && group % 128 != 0;
+  const int G = wbits == 4 ? (int)(K / group) : 0;
+  int tm, tn;
+  pick_small_tile(M, N, K, G, wbits, s64, split, ssz, tm, tn);
+  const int xp = wbits == 4 && !s64 ? 4 : 2;
+  const bool slices = 4 * tm * tn + 8 * (tm * xp + tn) <= 112 && 8 * tm * tn <= 128 &&
+                      small_xls_fits(K, G, wbits, s64, tm, tn, ssz);
+  const float rounds = (float)cdiv(cdiv(M, 16 * tm) * cdiv(N, 16 * tn), 256);
+  const float mb = (float)small_cost(M, N, K, wbits, tm, tn) * 1e-6f, mf = rounds * (float)K * (float)(tm * tn) * 1e-4f;
+  if (wbits == 4) return slices ? 0.4f + 7.8f * mb + 3.0f * mf + 2.7f * rounds : 3.2f + 26.5f * mb + 0.93f * mf + 0.37f * rounds;
+  return slices ? 2.9f + 6.5f * mb + 2.74f * mf + 0.6f * rounds : 2.4f + 22.8f * mb + 0.69f * mf + 1.24f * rounds;
 }
 
 int launch_gemm_small(int wbits, const WqArgs& p) { return small_impl(wbits, p, 0); }

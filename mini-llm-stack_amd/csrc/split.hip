@@ -52,7 +52,65 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   *reinterpret_cast<uint4*>(x2 + (int64_t)split_row(m, 1) * K + k0) = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
+// Three parts: hi = x truncated to bf16, mid = x - hi truncated to bf16, lo = the rest. Each
+// takes 8 of the 24 significant bits (the differences are exact in fp32), so the three add up
+// to x exactly. Non-finite x: hi = x, the others 0. Row m's part t is row 48 (m / 16) +
+// 16 t + m % 16.
+template <bool VEC>
+__global__ __launch_bounds__(256) void split_rows3_kernel(const float* __restrict__ x, int64_t ldx, int M, int K,
+                                                          __bf16* __restrict__ x2, int Mp) {
+  const int64_t pieces = K / 8;
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= pieces * Mp) return;
+  const int m = (int)(t / pieces), k0 = (int)(t % pieces) * 8;
+  float v[8];
+  if (m < M) {
+    if constexpr (VEC) {
+      const float4 a = *reinterpret_cast<const float4*>(x + (int64_t)m * ldx + k0);
+      const float4 b = *reinterpret_cast<const float4*>(x + (int64_t)m * ldx + k0 + 4);
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = x[(int64_t)m * ldx + k0 + e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+  }
+  uint32_t h[4], d[4], l[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float h0, h1, r0, r1, d0, d1, l0, l1;
+    split_f32(v[2 * q], h0, r0);
+    split_f32(v[2 * q + 1], h1, r1);
+    split_f32(r0, d0, l0);
+    split_f32(r1, d1, l1);
+    h[q] = pack2_bits((__bf16)h0, (__bf16)h1);  // (all exact)
+    d[q] = pack2_bits((__bf16)d0, (__bf16)d1);
+    l[q] = pack2_bits((__bf16)l0, (__bf16)l1);
+  }
+  __bf16* dst = x2 + (int64_t)(48 * (m >> 4) + (m & 15)) * K + k0;
+  *reinterpret_cast<uint4*>(dst) = make_uint4(h[0], h[1], h[2], h[3]);
+  *reinterpret_cast<uint4*>(dst + (int64_t)16 * K) = make_uint4(d[0], d[1], d[2], d[3]);
+  *reinterpret_cast<uint4*>(dst + (int64_t)32 * K) = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
 }  // namespace
+
+int launch_split_parts(const float* x, int64_t ldx, int64_t M, int64_t K, int parts, void* x2, hipStream_t st) {
+  if (parts == 2) return launch_split_rows(x, ldx, M, K, x2, st);
+  if (parts != 3 || K % 8 != 0 || !aligned(x2, 16)) return MLS_ERR_UNSUPPORTED;
+  const int64_t Mp = cdiv(M, 16) * 16;
+  const int64_t threads = Mp * (K / 8);
+  if (Mp > 0x3FFFFFFF || K > 0x3FFFFFFF || cdiv(threads, 256) > 0x7FFFFFFF) return MLS_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)cdiv(threads, 256));
+  if (aligned(x, 16) && ldx % 4 == 0)
+    hipLaunchKernelGGL(split_rows3_kernel<true>, grid, dim3(256), 0, st, x, ldx, (int)M, (int)K, (__bf16*)x2, (int)Mp);
+  else
+    hipLaunchKernelGGL(split_rows3_kernel<false>, grid, dim3(256), 0, st, x, ldx, (int)M, (int)K, (__bf16*)x2, (int)Mp);
+  return check_launch("split rows");
+}
 
 int launch_split_rows(const float* x, int64_t ldx, int64_t M, int64_t K, void* x2, hipStream_t st) {
   if (K % 8 != 0 || !aligned(x2, 16)) return MLS_ERR_UNSUPPORTED;

@@ -40,6 +40,9 @@ int launch_gemv_mfma_f32(int wbits, const WqArgs& p);
 // Small / medium GEMM for 16-bit activations (MFMA operands straight into registers, K
 // split over a block's wavefronts). MLS_ERR_UNSUPPORTED outside its fast path.
 int launch_gemm_small(int wbits, const WqArgs& p);
+// Its time for a shape in us, by a fitted model (ssz: bytes of a scale; split: M counts the
+// rows of the split matrix).
+float small_estimate_us(int wbits, int64_t M, int64_t N, int64_t K, int group, int ssz, bool split);
 
 // MFMA tiled GEMM for 16-bit activations. MLS_ERR_UNSUPPORTED outside its fast path.
 int launch_gemm_wq_mfma(int wbits, const WqArgs& p);
@@ -57,6 +60,10 @@ int launch_gemv_mfma_split(int wbits, const WqArgs& p);
 int launch_gemm_wq_mfma_split(int wbits, const WqArgs& p, int64_t m_out);
 // x fp32 [M][ldx] -> split rows [split_rows(M)][K] bf16 (zeros for rows past M).
 int launch_split_rows(const float* x, int64_t ldx, int64_t M, int64_t K, void* x2, hipStream_t st);
+// x fp32 [M][ldx] -> `parts` (2 or 3) bf16 rows per row, row m's part t at row
+// 16 parts (m / 16) + 16 t + m % 16 of x2 [16 parts ceil(M / 16)][K] (zeros past M): hi + lo
+// (x to 2^-16), or three parts that add up to x exactly.
+int launch_split_parts(const float* x, int64_t ldx, int64_t M, int64_t K, int parts, void* x2, hipStream_t st);
 // The GEMM of split rows q.a ([q.M][q.lda] bf16, q.M = split_rows(m_out)) into fp32 q.c:
 // the medium GEMM where the engine would have few tiles, else the engine.
 int launch_split_gemm(int wbits, const WqArgs& q, int64_t m_out);

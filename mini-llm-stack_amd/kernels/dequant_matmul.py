@@ -44,9 +44,9 @@ def int8_matmul(a: torch.Tensor, w_q: torch.Tensor, scale: torch.Tensor):
     lib = kernels.lib()
     # fp32 activations with M >= 2 run on the matrix cores as bf16 hi + lo parts, split
     # into a workspace from torch's caching allocator; other calls need none
-    need = lib.mls_wq_gemm_workspace(8, M, N, K, adt, 0)
+    need = lib.mlsx_wq_workspace(8, M, N, K, adt, 0)
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    kernels.check(lib.mls_int8_gemm_ws(
+    kernels.check(lib.mlsx_int8_gemm(
         a.data_ptr(), adt, ld(a), w_q.data_ptr(), ld(w_q), s.data_ptr(), sdt,
         c.data_ptr(), adt, ld(c), M, N, K, ws.data_ptr() if need else None, need, stream(dev)), "int8_matmul")
     return c
@@ -98,9 +98,9 @@ def int4_matmul(a: torch.Tensor, w_packed: torch.Tensor, scale: torch.Tensor,
     sdt = dt_code(scale.dtype, "int4_matmul scale")
     c = torch.empty(M, N, dtype=a.dtype, device=dev)
     lib = kernels.lib()
-    need = lib.mls_wq_gemm_workspace(4, M, N, K, adt, group_size)
+    need = lib.mlsx_wq_workspace(4, M, N, K, adt, group_size)
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
-    kernels.check(lib.mls_int4_gemm_ws(
+    kernels.check(lib.mlsx_int4_gemm(
         a.data_ptr(), adt, ld(a), w_packed.data_ptr(), ld(w_packed),
         scale.data_ptr(), sdt, scale.stride(0), scale.stride(1), group_size,
         c.data_ptr(), adt, ld(c), M, N, K, ws.data_ptr() if need else None, need, stream(dev)), "int4_matmul")
