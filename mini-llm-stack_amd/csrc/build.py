@@ -22,7 +22,7 @@ CSRC = Path(__file__).resolve().parent
 PKG = CSRC.parent
 OUT = PKG / "libmls_hip.so"
 BUILD = CSRC / "_build"
-SOURCES = ["abi.hip", "e4m3.hip", "quant.hip", "gemv.hip", "gemv_mfma.hip", "gemv_mfma8.hip", "gemm_mfma16.hip", "gemm_grouped.hip",
+SOURCES = ["abi.hip", "e4m3.hip", "quant.hip", "gemv.hip", "gemv_mfma.hip", "gemv_mfma8.hip", "gemm_mfma16.hip", "gemm_grouped.hip", "grouped_skinny.hip",
            "wq_abi.hip", "gemm_small.hip", "gemm_ksplit.hip", "gemm_bytes.hip", "gemm_fp8.hip", "dgrad.hip", "moe.hip", "transpose.hip", "paged_attn.hip", "split.hip"]
 ARCH = "gfx950"
 # Per-source device-code options.
@@ -44,6 +44,7 @@ EXTRA_FLAGS = {"gemv.hip": PRELOAD,
                "gemv_mfma8.hip": PRELOAD,
                "gemm_small.hip": VGPR_FORM + PRELOAD,
                "gemm_grouped.hip": VGPR_FORM,
+               "grouped_skinny.hip": VGPR_FORM,
                "split.hip": PRELOAD}
 
 

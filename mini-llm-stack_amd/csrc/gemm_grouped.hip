@@ -515,7 +515,12 @@ int grouped_splits(int64_t M, int E, int64_t N, int64_t K, int group) {
       if (tiles * s >= 512) break;  // two blocks per CU reached
     }
   }
-  return env > 0 ? 1 : best;
+  if (env > 0) return 1;
+  // few rows an expert (grouped_skinny.hip): a block's wavefronts share a range, so ranges of at
+  // least 8 steps of 128 k (512 -> 128 k a wavefront: 11.1 us against 9.6 unsplit to that point)
+  if (M <= (int64_t)E * 8)
+    while (best > 2 && K / best < 1024) best /= 2;
+  return best;
 }
 
 template <int SCL>
@@ -537,6 +542,10 @@ int launch_grouped_partial(const Mfma16Params& p, hipStream_t st, bool bf16) {
   if (s < 1 || p.K % s != 0) return MLS_ERR_UNSUPPORTED;
   const int64_t kp = p.K / s, G = kp / p.group;
   if (kp % 64 != 0 || kp % p.group != 0) return MLS_ERR_UNSUPPORTED;
+  if (grouped_skinny_fits(p, false)) {
+    const int rc = launch_grouped_skinny(p, st, bf16, false, true);
+    if (rc != MLS_ERR_UNSUPPORTED) return rc;
+  }
   const int tmx = chunk_tmx(p.M, p.E);
   const bool stab = p.s_dt == MLS_F16 && p.ld_sg == 1 && G % 4 == 0 && G <= 32 && (p.ld_sn % 4) == 0 &&
                     (p.s_estride % 4) == 0 && aligned(p.s, 8);
@@ -546,6 +555,12 @@ int launch_grouped_partial(const Mfma16Params& p, hipStream_t st, bool bf16) {
 }
 
 int launch_grouped_seg(const Mfma16Params& p, hipStream_t st, bool bf16, bool gate_up) {
+  Mfma16Params one = p;
+  one.ksplit = 1;
+  if (grouped_skinny_fits(one, gate_up)) {
+    const int rc = launch_grouped_skinny(one, st, bf16, gate_up, false);
+    if (rc != MLS_ERR_UNSUPPORTED) return rc;
+  }
   const int tmx = chunk_tmx(p.M, p.E);
   // scale table in LDS: fp16 scales, contiguous groups, G a multiple of 4 up to 128,
   // 8-byte aligned rows; a table of up to 32 groups keeps two blocks per CU

@@ -209,6 +209,10 @@ int launch_grouped_seg(const Mfma16Params& p, hipStream_t st, bool bf16, bool ga
 // partial s at p.c + s * p.c_sstride). MLS_ERR_UNSUPPORTED unless each range is a
 // multiple of 64 and of the group and its scales fit the 32-group LDS table.
 int launch_grouped_partial(const Mfma16Params& p, hipStream_t st, bool bf16);
+// The grouped kernel for few rows an expert (grouped_skinny.hip); p.ksplit >= 1, partial: fp32
+// partial products of p.ksplit K ranges.
+bool grouped_skinny_fits(const Mfma16Params& p, bool gate_up);
+int launch_grouped_skinny(const Mfma16Params& p, hipStream_t st, bool bf16, bool gate_up, bool partial);
 // K splits that give the down projection of an expert MLP (few column tiles) two
 // blocks per CU; 1 when no split is needed or possible.
 int grouped_splits(int64_t M, int E, int64_t N, int64_t K, int group);
