@@ -28,6 +28,24 @@ int mlsx_int4_gemm(const void* a, int a_dt, int64_t lda, const uint8_t* w, int64
                    int64_t ld_sn, int64_t ld_sg, int group, void* c, int c_dt, int64_t ldc, int64_t M, int64_t N,
                    int64_t K, void* workspace, int64_t ws_bytes, mls_stream_t stream);
 
+/* ---------------------------------------------------------------- MoE routing */
+
+/* Top-k of softmax(logits[t]) in fp32, largest first, divided by their sum (train/model.py:
+ * 158-162): weights fp32 [tokens][k], experts int64 [tokens][k]. logits: dt [tokens][ld]. At most
+ * 256 experts and k = 8 (MLS_ERR_UNSUPPORTED above). */
+int mlsx_route_topk(const void* logits, int dt, int64_t ld, int64_t tokens, int E, int k, float* weights,
+                    int64_t* experts, mls_stream_t stream);
+
+/* The expert-sorted order of n = tokens * k assignments (kernels/moe_routing.py:116-130), stable:
+ * token_of_slot[p] (int32 [n]) the token of sorted row p, seg_off (int32 [E + 1]) the segments,
+ * pos[i] (int64 [n]) the sorted row of assignment i. An id outside [0, E) joins no segment (pos
+ * -1; rows past the last segment hold token -1) and sets *bad (1, or 2 where one is negative; 0
+ * otherwise), which may be pinned host memory. At most 256 experts and MLSX_ROUTE_MAX
+ * assignments. */
+#define MLSX_ROUTE_MAX 32768
+int mlsx_route_sort(const int64_t* experts, int64_t n, int k, int E, int32_t* token_of_slot, int32_t* seg_off,
+                    int64_t* pos, int32_t* bad, mls_stream_t stream);
+
 /* ---------------------------------------------------------------- FP8 training */
 
 /* The fp8 operands of train/fp8.py:62-95 padded for the K-contiguous GEMM:

@@ -4,7 +4,9 @@
 // A position outside [0, x_rows) contributes nothing (it is never dereferenced).
 // x may hold `splits` partial products of a K-split GEMM (fp32, split_stride apart):
 // they are summed per row before the weighting, and the output dtype is separate.
-// HBM-bound: k rows read, one row written; 16-byte vector accesses when the rows allow.
+// HBM-bound: k rows read, one row written; 16-byte vector accesses when the rows allow. The
+// columns of a token are spread over blocks too (grid.y), so that a decode batch of 16 tokens is
+// more than 16 blocks.
 #include <type_traits>
 
 #include "common.h"
@@ -44,7 +46,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const T* __restrict__ 
     // 8 elements per thread and step: one 16-byte access of 16-bit data, two of fp32,
     // four of fp64 (rows and d are multiples of 8 elements, so every access is aligned)
     constexpr int V = 8, XQ = V * (int)sizeof(T) / 16, OQ = V * (int)sizeof(OT) / 16;
-    for (int64_t d = (int64_t)threadIdx.x * V; d < D; d += (int64_t)blockDim.x * V) {
+    for (int64_t d = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * V; d < D;
+         d += (int64_t)gridDim.y * blockDim.x * V) {
       A acc[V];
 #pragma unroll
       for (int i = 0; i < V; ++i) acc[i] = 0;
@@ -74,7 +77,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const T* __restrict__ 
         reinterpret_cast<uint4*>(out + t * ldo + d)[q] = reinterpret_cast<const uint4*>(o)[q];
     }
   } else {
-    for (int64_t d = threadIdx.x; d < D; d += blockDim.x) {
+    for (int64_t d = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; d < D; d += (int64_t)gridDim.y * blockDim.x) {
       A acc = 0;
       for (int s = 0; s < k; ++s) {
         const int64_t r = pos[t * k + s];
@@ -94,7 +97,10 @@ int launch_combine(const void* x, int64_t ldx, int64_t x_rows, int splits, int64
                    hipStream_t st) {
   const bool vec = D % 8 == 0 && ldx % 8 == 0 && ldo % 8 == 0 && sstride % 8 == 0 && aligned(x, 16) &&
                    aligned(out, 16);
-  const dim3 grid((unsigned)T_), block(256);
+  // one pass of the columns a block; fewer threads a block where tokens are few
+  const int threads = T_ < 256 ? 64 : 256;
+  const int64_t ny = cdiv(D, (vec ? 8 : 1) * (int64_t)threads);
+  const dim3 grid((unsigned)T_, (unsigned)(ny < 1024 ? ny : 1024)), block((unsigned)threads);
 #define MLS_COMBINE(WT)                                                                                   \
   hipLaunchKernelGGL((moe_combine_kernel<T, WT, OT>), grid, block, 0, st, (const T*)x, ldx, x_rows, splits, \
                      sstride, (const WT*)w, pos, k, (OT*)out, ldo, D, vec)

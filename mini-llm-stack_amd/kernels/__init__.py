@@ -99,10 +99,14 @@ SIGNATURES = {
 
 # include/mls_ext.h: entry points of this package's own modules
 ABSMAX_PARTS = 1024  # MLSX_ABSMAX_PARTS
+ROUTE_MAX = 32768  # MLSX_ROUTE_MAX
+ROUTE_MAX_EXPERTS, ROUTE_MAX_TOP = 256, 8
 EXT_SIGNATURES = {
     "mlsx_wq_workspace": ([_I, _I64, _I64, _I64, _I, _I], _I64),
     "mlsx_int8_gemm": (SIGNATURES["mls_int8_gemm_ws"][0], _I),
     "mlsx_int4_gemm": (SIGNATURES["mls_int4_gemm_ws"][0], _I),
+    "mlsx_route_topk": ([_P, _I, _I64, _I64, _I, _I, _P, _P, _P], _I),
+    "mlsx_route_sort": ([_P, _I64, _I, _I, _P, _P, _P, _P, _P], _I),
     "mlsx_fp8_encode_pad": ([_I, _P, _I, _I64, _I64, _I64, _F, _P, _I64, _P, _P, _P], _I),
     "mlsx_absmax_parts": ([_P, _I, _I64, _P, _P], _I),
     "mlsx_absmax_scales": ([_P, _I, _F, _P, _P, _P], _I),

@@ -56,3 +56,11 @@ def scale_vector(scale: torch.Tensor) -> tuple[torch.Tensor, int]:
     if scale.dtype not in (torch.float32, torch.float16):
         scale = scale.to(torch.float32)
     return scale, _DT[scale.dtype]
+
+
+def plain(t: torch.Tensor) -> bool:
+    """An ordinary device tensor outside tracing and function transforms, from which no gradient
+    is asked for: one whose memory a kernel may read in place of differentiable torch ops."""
+    return (type(t) is torch.Tensor and t.device.type == "cuda" and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0)

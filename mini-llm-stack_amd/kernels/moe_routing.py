@@ -24,11 +24,24 @@ from __future__ import annotations
 import torch
 
 import kernels
-from kernels._hip import dt_code, ld, require_hip, stream
+from kernels._hip import dt_code, ld, plain, require_hip, stream
+
+
+_ROUTE_DT = (torch.float32, torch.float16, torch.bfloat16)
 
 
 def route_topk(logits: torch.Tensor, k: int):
     """(weights [T, k] fp32, experts [T, k] int64)."""
+    if (plain(logits) and logits.dim() == 2 and logits.dtype in _ROUTE_DT and logits.stride(1) == 1
+            and 0 < k <= min(logits.shape[1], kernels.ROUTE_MAX_TOP) and logits.shape[1] <= kernels.ROUTE_MAX_EXPERTS
+            and logits.stride(0) >= logits.shape[1]):
+        T, E = logits.shape
+        weights = torch.empty(T, k, dtype=torch.float32, device=logits.device)
+        experts = torch.empty(T, k, dtype=torch.int64, device=logits.device)
+        kernels.check(kernels.lib().mlsx_route_topk(
+            logits.data_ptr(), dt_code(logits.dtype, "route_topk"), logits.stride(0), T, E, k, weights.data_ptr(),
+            experts.data_ptr(), stream(logits.device)), "route_topk")
+        return weights, experts
     probs = torch.softmax(logits.float(), dim=-1)
     weights, experts = torch.topk(probs, k, dim=-1)
     weights = weights / weights.sum(dim=-1, keepdim=True)
@@ -44,6 +57,41 @@ def sort_by_expert(experts_idx: torch.Tensor, n_experts: int):
     pos = torch.empty_like(order)
     pos[order] = torch.arange(T * k, device=flat.device)
     return order // k, counts, pos.reshape(T, k)
+
+
+class _Route:
+    """sort_by_expert in one launch, as the grouped kernels take it: token_of_slot (int32), the
+    segment offsets (int32 [E + 1]) and pos (int64 [T, k]). check() raises for expert ids outside
+    [0, E), which the kernel leaves out; it waits for that launch alone, so the caller
+    enqueues the layer's GEMMs first."""
+
+    @staticmethod
+    def takes(experts_idx: torch.Tensor, n_experts: int) -> bool:
+        return (plain(experts_idx) and experts_idx.dim() == 2 and experts_idx.dtype in (torch.int64, torch.int32)
+                and 0 < experts_idx.numel() <= kernels.ROUTE_MAX and 0 < n_experts <= kernels.ROUTE_MAX_EXPERTS)
+
+    def __init__(self, experts_idx: torch.Tensor, n_experts: int):
+        dev = experts_idx.device
+        idx = experts_idx.to(torch.int64).contiguous()
+        n = idx.numel()
+        ints = torch.empty(n + n_experts + 1, dtype=torch.int32, device=dev)
+        self.token_of_slot, self.seg_off = ints[:n], ints[n:]
+        self.pos = torch.empty(idx.shape, dtype=torch.int64, device=dev)
+        self.bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        kernels.check(kernels.lib().mlsx_route_sort(
+            idx.data_ptr(), n, idx.shape[1], n_experts, self.token_of_slot.data_ptr(), self.seg_off.data_ptr(),
+            self.pos.data_ptr(), self.bad.data_ptr(), stream(dev)), "moe_dispatch_combine")
+        self.done = torch.cuda.Event()
+        self.done.record(torch.cuda.current_stream(dev))
+        self.n_experts = n_experts
+
+    def check(self) -> None:
+        self.done.synchronize()
+        bad = int(self.bad)
+        if bad == 2:
+            raise RuntimeError("moe_dispatch_combine: negative expert index")
+        if bad:
+            raise ValueError(f"moe_dispatch_combine: expert index past the {self.n_experts} experts")
 
 
 def gather_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
@@ -100,9 +148,17 @@ def moe_dispatch_combine(flat: torch.Tensor, weights: torch.Tensor, experts_idx:
     from serve.quantize import stacked_int4_experts
 
     n_experts = len(expert_modules)
-    token_of_slot, counts, pos = sort_by_expert(experts_idx, n_experts)
     st = stacked_int4_experts(expert_modules)
-    if st is not None and flat.dtype in (torch.bfloat16, torch.float16):
+    quantized = st is not None and flat.dtype in (torch.bfloat16, torch.float16)
+    if quantized and _Route.takes(experts_idx, n_experts):
+        route = _Route(experts_idx, n_experts)
+        out = int4_expert_mlp_combine(flat, route.seg_off, st["w_gate"][0], st["w_gate"][1], st["w_up"][0],
+                                      st["w_up"][1], st["w_down"][0], st["w_down"][1], st["group_size"], weights,
+                                      route.pos, a_rows=route.token_of_slot)
+        route.check()
+        return out
+    token_of_slot, counts, pos = sort_by_expert(experts_idx, n_experts)
+    if quantized:
         # the gather runs inside the gate/up kernel's activation load (a_rows)
         return int4_expert_mlp_combine(flat, segment_offsets(counts), st["w_gate"][0], st["w_gate"][1],
                                        st["w_up"][0], st["w_up"][1], st["w_down"][0], st["w_down"][1],
