@@ -28,6 +28,19 @@ int mlsx_int4_gemm(const void* a, int a_dt, int64_t lda, const uint8_t* w, int64
                    int64_t ld_sn, int64_t ld_sg, int group, void* c, int c_dt, int64_t ldc, int64_t M, int64_t N,
                    int64_t K, void* workspace, int64_t ws_bytes, mls_stream_t stream);
 
+/* ---------------------------------------------------------------- paged attention */
+
+/* mls_paged_attention_decode with the contexts cut into pieces of equal length instead of as
+ * many splits a sequence, so that a batch of unequal lengths keeps the GPU even. Arguments as
+ * there; the workspace holds mlsx_paged_attention_workspace floats (0: none). */
+int64_t mlsx_paged_attention_workspace(int64_t n_seqs, int64_t H, int64_t D, int64_t block_size, int64_t max_blocks);
+int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss, int64_t q_sh, const void* k_pool,
+                                const void* v_pool, int kv_dt, int64_t kv_sb, int64_t kv_sh, int64_t kv_st,
+                                int64_t num_blocks, const int32_t* block_tables, int64_t bt_ss, int64_t max_blocks,
+                                const int32_t* context_lens, void* out, int64_t o_ss, int64_t o_sh, int64_t n_seqs,
+                                int64_t H, int64_t D, int64_t block_size, float scale, float* workspace,
+                                int64_t workspace_floats, mls_stream_t stream);
+
 /* ---------------------------------------------------------------- MoE routing */
 
 /* Top-k of softmax(logits[t]) in fp32, largest first, divided by their sum (train/model.py:

@@ -82,7 +82,64 @@ struct PagedArgs {
   float scale;
   float* ws;  // splits > 1: [n_seqs][H][splits][D + 2] (acc[D], m, l)
   int splits;
+  int per;  // least table blocks of a piece (piece_blocks); 0: a sequence's blocks over `splits`
 };
+
+// Table blocks of a sequence's cached tokens, never past its table row.
+__device__ __forceinline__ int live_blocks(const PagedArgs& a, int ctx) {
+  return (int)min((int64_t)((max(ctx, 0) + a.BS - 1) / a.BS), a.max_blocks);
+}
+
+// Table blocks a piece, where contexts are cut into pieces of one length (a.per > 0): the length
+// that makes about 4096 pieces of the batch's own blocks, a.per (from the largest context the
+// tables allow) at least. Every wavefront of both kernels finds the same value: one load of
+// the lengths and a sum. Batches past 256 sequences take a.per.
+// (32 heads of 128, bf16, us: 40 sequences of 1 to 4096 tokens 98 as 4 splits a sequence, which
+// wait for the longest one's, 80 as pieces; 64 of 1 to 2048 tokens 92 and 70; all 2048 long 331
+// and 328. Eight heads, one sequence of 4096: 38 and 20, mostly the table's register.)
+__device__ __forceinline__ int piece_blocks(const PagedArgs& a, int lane) {
+  if (a.n_seqs > 256) return a.per;
+  int sum = 0;
+  for (int s0 = 0; s0 < a.n_seqs; s0 += 64)
+    if (s0 + lane < a.n_seqs) sum += live_blocks(a, a.ctx[s0 + lane]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  const int want = (int)min(((int64_t)sum * a.H + 4095) / 4096, (int64_t)0x3FFFFFFF);
+  return __builtin_amdgcn_readfirstlane(max(want, a.per));
+}
+
+// Table blocks [b0, b1) of split `split` of a sequence of nb blocks, and how many of its splits
+// hold any: as many even pieces of up to `piece` blocks as it takes (a split past them leaves at
+// once, and a sequence of one piece needs no merge), or, with piece = 0, a.splits even shares.
+__device__ __forceinline__ int split_range(const PagedArgs& a, int nb, int split, int piece, int& b0, int& b1) {
+  if (piece == 0) {
+    const int per = (nb + a.splits - 1) / a.splits;
+    b0 = split * per;
+    b1 = min(nb, b0 + per);
+    return a.splits;
+  }
+  const int live = max((nb + piece - 1) / piece, 1), per = (nb + live - 1) / live;
+  b0 = min(split * per, nb);  // (split < a.splits, so the product stays below twice the table)
+  b1 = min(nb, b0 + per);
+  return live;
+}
+
+// Wavefront item -> (split, head, sequence). Pieces of a fixed length: the pairs of one piece
+// index side by side (a block's four wavefronts do equal work, on neighbouring heads of the
+// same cache blocks), the pieces that few sequences reach last.
+__device__ __forceinline__ void item_of(const PagedArgs& a, int64_t item, int& split, int& head, int& seq) {
+  int64_t pair;
+  if (a.per == 0) {
+    split = (int)(item % a.splits);
+    pair = item / a.splits;
+  } else {
+    const int64_t pairs = (int64_t)a.n_seqs * a.H;
+    split = (int)(item / pairs);
+    pair = item - split * pairs;
+  }
+  head = (int)(pair % a.H);
+  seq = (int)(pair / a.H);
+}
 
 template <typename QT, typename KT, int CPT>
 __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
@@ -94,21 +151,25 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
   if (item >= items) return;
   // wave-uniform indices (readfirstlane), so table entries and lengths are scalar
   // loads, outside the vector-load counter that paces the K/V prefetch
-  const int split = __builtin_amdgcn_readfirstlane((int)(item % a.splits));
-  const int head = __builtin_amdgcn_readfirstlane((int)((item / a.splits) % a.H));
-  const int seq = __builtin_amdgcn_readfirstlane((int)(item / ((int64_t)a.splits * a.H)));
+  int split, head, seq;
+  item_of(a, item, split, head, seq);
+  split = __builtin_amdgcn_readfirstlane(split);
+  head = __builtin_amdgcn_readfirstlane(head);
+  seq = __builtin_amdgcn_readfirstlane(seq);
   const int ts = lane / CPT, part = lane % CPT;
+  const int32_t* table = a.bt + (int64_t)seq * a.bt_ss;
 
+  const int ctx = a.ctx[seq];
+  const int nb = live_blocks(a, ctx);
+  int b0, b1;
+  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  if (split >= live) return;
   float q[EPC];
   {
     const QT* qp = static_cast<const QT*>(a.q) + seq * a.q_ss + head * a.q_sh + part * EPC;
 #pragma unroll
     for (int e = 0; e < EPC; ++e) q[e] = to_f32(qp[e]);
   }
-  const int ctx = a.ctx[seq];
-  const int nb = (int)min((int64_t)((max(ctx, 0) + a.BS - 1) / a.BS), a.max_blocks);  // never past the table row
-  const int per = (nb + a.splits - 1) / a.splits;
-  const int b0 = split * per, b1 = min(nb, b0 + per);
 
   float m = NEG_INF, l = 0.0f, acc[EPC];
 #pragma unroll
@@ -123,11 +184,32 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
   const int total = a.num_blocks > 0 ? (b1 - b0) * spb : 0;
   const KT* kbase = static_cast<const KT*>(a.kp) + head * a.kv_sh + part * EPC;
   const KT* vbase = static_cast<const KT*>(a.vp) + head * a.kv_sh + part * EPC;
-  const int32_t* table = a.bt + (int64_t)seq * a.bt_ss;
-  auto issue = [&](int step, uint4 (&kr)[UNR], uint4 (&vr)[UNR], bool& ok) __attribute__((always_inline)) {
-    const int b = b0 + step / spb, t0 = (step % spb) * UNR * TPI;
-    const int blk = table[b];
-    ok = blk >= 0 && blk < a.num_blocks;  // uniform over the wavefront
+  // the next step to issue: block ib of the table, token it of it (kept as counters: a division a
+  // step costs more than the step's other scalar work). The table entries of up to 64 blocks
+  // sit in a register, a lane each, so that no load waits for a table entry's own latency.
+  struct Step {
+    int b, t0;
+    bool ok;  // uniform over the wavefront
+  };
+  int ib = b0, it = 0, left = total, tb = b0;
+  int tabv = total > 0 ? table[min(tb + lane, b1 - 1)] : -1;
+  auto issue = [&](uint4 (&kr)[UNR], uint4 (&vr)[UNR], Step& st) __attribute__((always_inline)) {
+    if (ib - tb >= 64) {
+      tb = ib;
+      tabv = table[min(tb + lane, b1 - 1)];
+      __builtin_amdgcn_s_waitcnt(0 | 0x70 | 0xF00);  // (once in 64 blocks)
+    }
+    const int blk = __builtin_amdgcn_readlane(tabv, ib - tb);
+    const int t0 = it;
+    const bool ok = left > 0 && blk >= 0 && blk < a.num_blocks;
+    st = Step{ib, t0, ok};
+    if (--left > 0) {
+      it += UNR * TPI;
+      if (it >= a.BS) {
+        it = 0;
+        ++ib;
+      }
+    }
     // unconditional loads (a branch around them would make the compiler wait for
     // each): an invalid block reads block 0, a slot past the block end reads the
     // block's last token; score() gives both weight 0
@@ -141,8 +223,9 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
       vr[u] = __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const kv16_t*>(vbase + boff + t * a.kv_st)));
     }
   };
-  auto score = [&](int step, const uint4 (&kr)[UNR], const uint4 (&vr)[UNR], bool ok) __attribute__((always_inline)) {
-    const int b = b0 + step / spb, t0 = (step % spb) * UNR * TPI;
+  auto score = [&](const uint4 (&kr)[UNR], const uint4 (&vr)[UNR], const Step& st) __attribute__((always_inline)) {
+    const int b = st.b, t0 = st.t0;
+    const bool ok = st.ok;
     float sc[UNR];
     float mx = m;
 #pragma unroll
@@ -175,15 +258,14 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
     m = mx;
   };
   uint4 ka[UNR], va[UNR], kb[UNR], vb[UNR];
-  bool oka = false, okb = false;
-  // branch-free pairs of steps: the step indices are clamped (a repeated last step is
-  // loaded again and scored with weight 0)
-  if (total > 0) issue(0, ka, va, oka);
+  Step sa{0, 0, false}, sb{0, 0, false};
+  // branch-free pairs of steps: past the last one it is loaded again and scored with weight 0
+  if (total > 0) issue(ka, va, sa);
   for (int step = 0; step < total; step += 2) {
-    issue(min(step + 1, total - 1), kb, vb, okb);
-    score(step, ka, va, oka);
-    issue(min(step + 2, total - 1), ka, va, oka);
-    score(step + 1, kb, vb, okb && step + 1 < total);
+    issue(kb, vb, sb);
+    score(ka, va, sa);
+    issue(ka, va, sa);
+    score(kb, vb, sb);
   }
   // merge the token slots that share this lane's chunk (lanes part, part + CPT, ...)
 #pragma unroll
@@ -195,7 +277,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
     merge_state<EPC>(m, l, acc, m2, l2, acc2);
   }
   if (ts != 0) return;
-  if (a.splits == 1) {
+  if (live == 1) {
     const float inv = l == 0.0f ? 1.0f : 1.0f / l;
     QT* op = static_cast<QT*>(a.out) + seq * a.o_ss + head * a.o_sh + part * EPC;
 #pragma unroll
@@ -218,17 +300,17 @@ __global__ __launch_bounds__(256) void paged_attn_generic_kernel(const PagedArgs
   const int lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= (int64_t)a.n_seqs * a.H * a.splits) return;
-  const int split = (int)(item % a.splits);
-  const int head = (int)((item / a.splits) % a.H);
-  const int seq = (int)(item / ((int64_t)a.splits * a.H));
+  int split, head, seq;
+  item_of(a, item, split, head, seq);
   float q[4], acc[4] = {0.f, 0.f, 0.f, 0.f};
   const QT* qp = static_cast<const QT*>(a.q) + seq * a.q_ss + head * a.q_sh;
 #pragma unroll
   for (int i = 0; i < 4; ++i) q[i] = lane + 64 * i < a.D ? to_f32(qp[lane + 64 * i]) : 0.0f;
   const int ctx = a.ctx[seq];
-  const int nb = (int)min((int64_t)((max(ctx, 0) + a.BS - 1) / a.BS), a.max_blocks);  // never past the table row
-  const int per = (nb + a.splits - 1) / a.splits;
-  const int b0 = split * per, b1 = min(nb, b0 + per);
+  const int nb = live_blocks(a, ctx);
+  int b0, b1;
+  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  if (split >= live) return;
   float m = NEG_INF, l = 0.0f;
   const int32_t* table = a.bt + (int64_t)seq * a.bt_ss;
   for (int b = b0; b < b1; ++b) {
@@ -253,7 +335,7 @@ __global__ __launch_bounds__(256) void paged_attn_generic_kernel(const PagedArgs
       m = mn;
     }
   }
-  if (a.splits == 1) {
+  if (live == 1) {
     const float inv = l == 0.0f ? 1.0f : 1.0f / l;
     QT* op = static_cast<QT*>(a.out) + seq * a.o_ss + head * a.o_sh;
 #pragma unroll
@@ -271,30 +353,38 @@ __global__ __launch_bounds__(256) void paged_attn_generic_kernel(const PagedArgs
   }
 }
 
-// Merge the splits of one (sequence, head): one wavefront, lanes over D.
+// Merge the splits of one (sequence, head): one wavefront; lane s holds split s's maximum and
+// sum (at most 64 splits), then the lanes run over D with every split's factor broadcast.
 template <typename QT>
 __global__ __launch_bounds__(256) void paged_attn_merge_kernel(const PagedArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= (int64_t)a.n_seqs * a.H) return;
-  const int head = (int)(item % a.H), seq = (int)(item / a.H);
+  const int head = (int)(item % a.H), seq = __builtin_amdgcn_readfirstlane((int)(item / a.H));
+  const int nb = live_blocks(a, a.ctx[seq]);
+  int b0, b1;
+  const int live = split_range(a, nb, 0, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  if (live == 1) return;  // written by its only split
   const float* w = a.ws + item * a.splits * (a.D + 2);
-  float M = NEG_INF;
-  for (int s = 0; s < a.splits; ++s) M = fmaxf(M, w[s * (a.D + 2) + a.D]);
-  float L = 0.0f;
-  for (int s = 0; s < a.splits; ++s) {
-    const float ms = w[s * (a.D + 2) + a.D];
-    L += M == NEG_INF ? 0.0f : w[s * (a.D + 2) + a.D + 1] * __expf(ms - M);
-  }
+  const float ms = lane < live ? w[lane * (a.D + 2) + a.D] : NEG_INF;
+  const float ls = lane < live ? w[lane * (a.D + 2) + a.D + 1] : 0.0f;
+  const float M = wave_max(ms);
+  const float f = M == NEG_INF || ms == NEG_INF ? 0.0f : __expf(ms - M);
+  const float L = wave_sum(ls * f);
   const float inv = L == 0.0f ? 1.0f : 1.0f / L;
   QT* op = static_cast<QT*>(a.out) + seq * a.o_ss + head * a.o_sh;
-  for (int d = lane; d < a.D; d += 64) {
+  for (int d0 = 0; d0 < a.D; d0 += 64) {
+    const int d = d0 + lane;
+    const float* wd = w + min(d, a.D - 1);
     float acc = 0.0f;
-    for (int s = 0; s < a.splits; ++s) {
-      const float ms = w[s * (a.D + 2) + a.D];
-      if (M != NEG_INF) acc = fmaf(w[s * (a.D + 2) + d], __expf(ms - M), acc);
+    for (int s0 = 0; s0 < live; s0 += 8) {  // eight records' loads in flight
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = wd[min(s0 + i, live - 1) * (a.D + 2)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc = s0 + i < live ? fmaf(v[i], __shfl(f, s0 + i, 64), acc) : acc;
     }
-    op[d] = from_f32<QT>(acc * inv);
+    if (d < a.D) op[d] = from_f32<QT>(acc * inv);
   }
 }
 
@@ -308,6 +398,19 @@ int choose_splits(int64_t n_seqs, int64_t H, int64_t max_blocks) {
   s = s < cap ? s : cap;
   s = s > 1 ? s : 1;
   return (int)(s < 64 ? s : 64);
+}
+
+// The least piece length, in table blocks: 128 tokens, or more where that would make over 16384
+// wavefronts or 64 splits a sequence. (64 and 256 tokens against 128, us: 4 sequences of up to
+// 1000 tokens, 32 heads, 19.5 and 18.3 against 13.7; one of 4096, 8 heads, 37 and 25 against 26.)
+int choose_per(int64_t n_seqs, int64_t H, int64_t block_size, int64_t max_blocks) {
+  const int64_t tokens = max_blocks * block_size, items = n_seqs * H;
+  int64_t piece = cdiv(items * tokens, 16384);
+  piece = piece > 128 ? piece : 128;
+  int64_t per = cdiv(piece, block_size);
+  const int64_t least = cdiv(max_blocks, 64);
+  per = per > least ? per : least;
+  return (int)(per < 0x3FFFFFFF ? per : 0x3FFFFFFF);
 }
 
 template <typename QT, typename KT>
@@ -390,7 +493,7 @@ int paged_prepare(const char* fn, const void* q, int q_dt, int64_t q_ss, int64_t
   if (!fast && D > 256) return fail(MLS_ERR_UNSUPPORTED, "%s: head dim %lld needs 16-byte rows", fn, (long long)D);
   a = PagedArgs{q, q_ss, q_sh, k_pool, v_pool, kv_sb, kv_sh, kv_st, num_blocks, block_tables, bt_ss,
                 max_blocks, context_lens, out, o_ss, o_sh, (int)n_seqs, (int)H, (int)D, (int)block_size,
-                scale, nullptr, splits};
+                scale, nullptr, splits, 0};
   return MLS_OK;
 }
 
@@ -420,6 +523,42 @@ extern "C" int mls_paged_attention_decode(const void* q, int q_dt, int64_t q_ss,
   if (rc != MLS_OK || done) return rc;
   if (need > 0 && (!workspace || workspace_floats < need))
     return fail(MLS_ERR_ARG, "%s: workspace of %lld floats needed (mls_paged_attention_workspace)", fn,
+                (long long)need);
+  a.ws = workspace;
+  return paged_launch(a, q_dt, kv_dt, fast, cpt, (hipStream_t)stream);
+}
+
+extern "C" int64_t mlsx_paged_attention_workspace(int64_t n_seqs, int64_t H, int64_t D, int64_t block_size,
+                                                  int64_t max_blocks) {
+  if (n_seqs <= 0 || H <= 0 || D <= 0 || block_size <= 0 || max_blocks <= 0) return 0;
+  const int64_t s = cdiv(max_blocks, choose_per(n_seqs, H, block_size, max_blocks));
+  return s > 1 ? n_seqs * H * s * (D + 2) : 0;
+}
+
+extern "C" int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss, int64_t q_sh,
+                                           const void* k_pool, const void* v_pool, int kv_dt, int64_t kv_sb,
+                                           int64_t kv_sh, int64_t kv_st, int64_t num_blocks,
+                                           const int32_t* block_tables, int64_t bt_ss, int64_t max_blocks,
+                                           const int32_t* context_lens, void* out, int64_t o_ss, int64_t o_sh,
+                                           int64_t n_seqs, int64_t H, int64_t D, int64_t block_size, float scale,
+                                           float* workspace, int64_t workspace_floats, mls_stream_t stream) {
+  const char* fn = "mlsx_paged_attention_decode";
+  PagedArgs a{};
+  int64_t need = 0;
+  bool fast = false, done = false;
+  int cpt = 0;
+  int rc = paged_prepare(fn, q, q_dt, q_ss, q_sh, k_pool, v_pool, kv_dt, kv_sb, kv_sh, kv_st, num_blocks,
+                         block_tables, bt_ss, max_blocks, context_lens, out, o_ss, o_sh, n_seqs, H, D, block_size,
+                         scale, a, need, fast, cpt, done);
+  if (rc != MLS_OK || done) return rc;
+  a.splits = 1;
+  if (max_blocks > 0) {
+    a.per = choose_per(n_seqs, H, block_size, max_blocks);
+    a.splits = (int)cdiv(max_blocks, a.per);
+  }
+  need = a.splits > 1 ? n_seqs * H * a.splits * (D + 2) : 0;
+  if (need > 0 && (!workspace || workspace_floats < need))
+    return fail(MLS_ERR_ARG, "%s: workspace of %lld floats needed (mlsx_paged_attention_workspace)", fn,
                 (long long)need);
   a.ws = workspace;
   return paged_launch(a, q_dt, kv_dt, fast, cpt, (hipStream_t)stream);

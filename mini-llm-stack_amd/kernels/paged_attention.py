@@ -7,10 +7,9 @@ Same function, arguments and result as the reference (kernels/paged_attention.py
 written and counted); scale defaults to D^-0.5. Returns [n_seqs, H, D] in q's dtype.
 
 The kernel (csrc/paged_attn.hip) walks each sequence's block table and keeps an
-online softmax, one wavefront per (sequence, head, context split); with few
-(sequence, head) pairs and long tables the context is split over several wavefronts
-and merged by a second kernel through a workspace this wrapper allocates (its size
-comes from mls_paged_attention_workspace). Tokens at or past a sequence's context
+online softmax, one wavefront per (sequence, head, piece of the context); contexts are
+cut into pieces of one length (128 tokens or more) and merged by a second kernel through a
+workspace this wrapper allocates (its size comes from mlsx_paged_attention_workspace). Tokens at or past a sequence's context
 length weigh 0; a zero context gives a zero output.
 """
 
@@ -53,9 +52,9 @@ def paged_attention_decode(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.
                          f"{tuple(ctx.shape)} for {n_seqs} sequences")
     max_blocks = bt.shape[1]
     L = kernels.lib()
-    ws_n = L.mls_paged_attention_workspace(n_seqs, H, D, max_blocks)
+    ws_n = L.mlsx_paged_attention_workspace(n_seqs, H, D, block_size, max_blocks)
     ws = torch.empty(max(ws_n, 1), dtype=torch.float32, device=dev)
-    kernels.check(L.mls_paged_attention_decode(
+    kernels.check(L.mlsx_paged_attention_decode(
         q.data_ptr(), dt_code(q.dtype, "paged_attention_decode q"), q.stride(0), q.stride(1),
         k_pool.data_ptr(), v_pool.data_ptr(), dt_code(k_pool.dtype, "paged_attention_decode pools"),
         k_pool.stride(0), k_pool.stride(1), k_pool.stride(2), num_blocks,
