@@ -59,6 +59,17 @@ int mlsx_route_topk(const void* logits, int dt, int64_t ld, int64_t tokens, int 
 int mlsx_route_sort(const int64_t* experts, int64_t n, int k, int E, int32_t* token_of_slot, int32_t* seg_off,
                     int64_t* pos, int32_t* bad, mls_stream_t stream);
 
+/* ---------------------------------------------------------------- weight gradient */
+
+/* dw[N][K] = dy[M][N]^T x[M][K], all fp32 row-major (kernels/autograd_ops.py:132), as bf16 parts
+ * that add up to the fp32 values. M >= 1. The 16-byte aligned workspace holds
+ * mlsx_dw_fp32_workspace bytes (0: sizes it does not take, MLS_ERR_UNSUPPORTED). */
+int64_t mlsx_dw_fp32_workspace(int64_t M, int64_t N, int64_t K);
+/* 1 where mlsx_dw_fp32 is faster than an fp32 library product and its workspace at most 4 GiB. */
+int mlsx_dw_fp32_pays(int64_t M, int64_t N, int64_t K);
+int mlsx_dw_fp32(const float* dy, int64_t lddy, const float* x, int64_t ldx, float* dw, int64_t lddw, int64_t M,
+                 int64_t N, int64_t K, void* ws, int64_t ws_bytes, mls_stream_t stream);
+
 /* ---------------------------------------------------------------- FP8 training */
 
 /* The fp8 operands of train/fp8.py:62-95 padded for the K-contiguous GEMM:

@@ -23,7 +23,7 @@ PKG = CSRC.parent
 OUT = PKG / "libmls_hip.so"
 BUILD = CSRC / "_build"
 SOURCES = ["abi.hip", "e4m3.hip", "quant.hip", "gemv.hip", "gemv_mfma.hip", "gemv_mfma8.hip", "gemm_mfma16.hip", "gemm_grouped.hip", "grouped_skinny.hip",
-           "wq_abi.hip", "gemm_small.hip", "gemm_ksplit.hip", "gemm_bytes.hip", "gemm_fp8.hip", "dgrad.hip", "moe.hip", "moe_route.hip", "transpose.hip", "paged_attn.hip", "split.hip"]
+           "wq_abi.hip", "gemm_small.hip", "gemm_ksplit.hip", "gemm_bytes.hip", "gemm_dw.hip", "gemm_fp8.hip", "dgrad.hip", "moe.hip", "moe_route.hip", "transpose.hip", "paged_attn.hip", "split.hip"]
 ARCH = "gfx950"
 # Per-source device-code options.
 # - Kernel-argument preloading (gemv.hip, gemv_mfma*.hip, gemm_small.hip, split.hip, and
@@ -45,6 +45,7 @@ EXTRA_FLAGS = {"gemv.hip": PRELOAD,
                "gemm_small.hip": VGPR_FORM + PRELOAD,
                "gemm_grouped.hip": VGPR_FORM,
                "grouped_skinny.hip": VGPR_FORM,
+               "gemm_dw.hip": VGPR_FORM,
                "split.hip": PRELOAD}
 
 

@@ -109,6 +109,9 @@ EXT_SIGNATURES = {
     "mlsx_paged_attention_decode": (SIGNATURES["mls_paged_attention_decode"][0], _I),
     "mlsx_route_topk": ([_P, _I, _I64, _I64, _I, _I, _P, _P, _P], _I),
     "mlsx_route_sort": ([_P, _I64, _I, _I, _P, _P, _P, _P, _P], _I),
+    "mlsx_dw_fp32_workspace": ([_I64, _I64, _I64], _I64),
+    "mlsx_dw_fp32_pays": ([_I64, _I64, _I64], _I),
+    "mlsx_dw_fp32": ([_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P], _I),
     "mlsx_fp8_encode_pad": ([_I, _P, _I, _I64, _I64, _I64, _F, _P, _I64, _P, _P, _P], _I),
     "mlsx_absmax_parts": ([_P, _I, _I64, _P, _P], _I),
     "mlsx_absmax_scales": ([_P, _I, _F, _P, _P, _P], _I),

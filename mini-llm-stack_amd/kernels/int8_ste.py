@@ -8,15 +8,38 @@ unchanged and its Int8MatmulSTE binds this package's int8_matmul / int8_dgrad;
 this module serves callers without the checkout.
 
 Forward: y = int8_matmul(x, W_q, s). Backward: dx = int8_dgrad(dy, W_q, s) on the
-device, and the fp32 master weight receives dy^T @ x (a plain fp GEMM with nothing
-quantized in it).
+device, and the fp32 master weight receives dy^T @ x (nothing quantized in it), for fp32
+on the matrix cores at the sizes where that is faster than the library's fp32 product.
 """
 
 from __future__ import annotations
 
 import torch
 
+import kernels
+from kernels._hip import ld, plain, rows, stream
 from kernels.dequant_matmul import int8_dgrad, int8_matmul
+
+
+def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """dy [M, N]^T @ x [M, K]. The kernel takes ordinary fp32 tensors; what torch has to see (a
+    gradient of the gradient, tracing, autocast) and other dtypes are torch's."""
+    if (dy.dtype != torch.float32 or x.dtype != torch.float32 or dy.dim() != 2 or x.dim() != 2
+            or x.shape[0] != dy.shape[0] or not plain(dy) or not plain(x) or dy.device != x.device
+            or torch.is_autocast_enabled("cuda")):
+        return dy.t() @ x
+    M, N = dy.shape
+    K = x.shape[1]
+    lib = kernels.lib()
+    if not lib.mlsx_dw_fp32_pays(M, N, K):
+        return dy.t() @ x
+    dy, x = rows(dy), rows(x)
+    need = lib.mlsx_dw_fp32_workspace(M, N, K)
+    ws = torch.empty(need, dtype=torch.uint8, device=dy.device)
+    dw = torch.empty(N, K, dtype=torch.float32, device=dy.device)
+    kernels.check(lib.mlsx_dw_fp32(dy.data_ptr(), ld(dy), x.data_ptr(), ld(x), dw.data_ptr(), ld(dw), M, N, K,
+                                   ws.data_ptr(), need, stream(dy.device)), "weight gradient")
+    return dw
 
 
 class Int8MatmulSTE(torch.autograd.Function):
@@ -30,7 +53,7 @@ class Int8MatmulSTE(torch.autograd.Function):
         x, w_q, scale = ctx.saved_tensors
         dy = dy.contiguous()
         dx = int8_dgrad(dy, w_q, scale)
-        dw = dy.t() @ x
+        dw = _weight_grad(dy, x)
         return dx, None, None, dw
 
 
