@@ -24,14 +24,15 @@ from kernels.dequant_matmul import int8_dgrad, int8_matmul
 def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """dy [M, N]^T @ x [M, K]. The kernel takes ordinary fp32 tensors; what torch has to see (a
     gradient of the gradient, tracing, autocast) and other dtypes are torch's."""
-    if (dy.dtype != torch.float32 or x.dtype != torch.float32 or dy.dim() != 2 or x.dim() != 2
-            or x.shape[0] != dy.shape[0] or not plain(dy) or not plain(x) or dy.device != x.device
-            or torch.is_autocast_enabled("cuda")):
+    if dy.dtype != torch.float32 or x.dtype != torch.float32 or dy.dim() != 2 or x.dim() != 2:
         return dy.t() @ x
+    # the sizes first: a small step is bound by its host work (100 tokens, 512 x 512: all checks
+    # in front of the library's product 23.1 us, the product's own call 19.7)
     M, N = dy.shape
     K = x.shape[1]
     lib = kernels.lib()
-    if not lib.mlsx_dw_fp32_pays(M, N, K):
+    if (not lib.mlsx_dw_fp32_pays(M, N, K) or x.shape[0] != M or not plain(dy) or not plain(x)
+            or dy.device != x.device or torch.is_autocast_enabled("cuda")):
         return dy.t() @ x
     dy, x = rows(dy), rows(x)
     need = lib.mlsx_dw_fp32_workspace(M, N, K)
