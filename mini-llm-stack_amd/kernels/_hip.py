@@ -23,13 +23,14 @@ def require_hip(fn: str, *tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{fn}: expected tensors, got {type(t).__name__}")
-        if t.device.type != "cuda":
-            raise TypeError(f"{fn}: tensors must be on a HIP device (got {t.device}); "
+        d = t.device
+        if d.type != "cuda":
+            raise TypeError(f"{fn}: tensors must be on a HIP device (got {d}); "
                             "the gfx950 kernels have no CPU implementation")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"{fn}: tensors on different devices ({dev} and {t.device})")
+            dev = d
+        elif d != dev:
+            raise ValueError(f"{fn}: tensors on different devices ({dev} and {d})")
     return dev
 
 
@@ -47,7 +48,10 @@ def ld(t: torch.Tensor) -> int:
 
 
 def stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The calling thread's current stream on dev, a tensor's device (so it has an index). The
+    handle itself: torch.cuda.current_stream's Stream object takes 2.0 us a call to make, an
+    eighth of a small eager layer's host time."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def scale_vector(scale: torch.Tensor) -> tuple[torch.Tensor, int]:
