@@ -49,8 +49,8 @@ def ld(t: torch.Tensor) -> int:
 
 def stream(dev: torch.device) -> int:
     """The calling thread's current stream on dev, a tensor's device (so it has an index). The
-    handle itself: torch.cuda.current_stream's Stream object takes 2.0 us a call to make, an
-    eighth of a small eager layer's host time."""
+    handle itself, 0.2 us a call: making torch.cuda.current_stream's Stream object takes 2.0
+    (an eager INT8 layer, fp32, 8 x 512 -> 2048: 18.4 -> 15.9 us)."""
     return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
