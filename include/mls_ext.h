@@ -41,6 +41,13 @@ int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss, int64_t q
                                 int64_t H, int64_t D, int64_t block_size, float scale, float* workspace,
                                 int64_t workspace_floats, mls_stream_t stream);
 
+/* ---------------------------------------------------------------- grouped INT4 GEMMs */
+
+/* 1 where the grouped INT4 entry points of mls.h take a call of M_total rows on the kernel for
+ * few rows an expert (grouped_skinny.hip), 0: on the chunk kernel, whose results it repeats bit
+ * for bit. splits: K ranges (1 but for the partial products). */
+int mlsx_int4_grouped_few_rows(int64_t M_total, int E, int64_t K, int group, int splits);
+
 /* ---------------------------------------------------------------- MoE routing */
 
 /* Top-k of softmax(logits[t]) in fp32, largest first, divided by their sum (train/model.py:

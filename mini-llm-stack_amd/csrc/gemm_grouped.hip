@@ -31,27 +31,6 @@
 
 namespace mls {
 
-namespace {
-
-// 32 INT4 weights (16 bytes, even k in the low nibble) -> 16 dwords of 16-bit floats
-// holding 16 (v - 8), k order.
-template <typename MT>
-__device__ __forceinline__ void widen_int4x16(const uint4& q, uint32_t* o) {
-  const uint32_t d[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const uint32_t x = d[t] ^ 0x88888888u;
-    const uint32_t hi = x & 0xF0F0F0F0u;         // k = 8t + 1, 3, 5, 7 (byte b: k = 8t + 2b + 1)
-    const uint32_t lo = (x << 4) & 0xF0F0F0F0u;  // k = 8t + 0, 2, 4, 6
-    o[4 * t + 0] = pack_exact2<MT>(sbyte_f32<0>(lo), sbyte_f32<0>(hi));
-    o[4 * t + 1] = pack_exact2<MT>(sbyte_f32<1>(lo), sbyte_f32<1>(hi));
-    o[4 * t + 2] = pack_exact2<MT>(sbyte_f32<2>(lo), sbyte_f32<2>(hi));
-    o[4 * t + 3] = pack_exact2<MT>(sbyte_f32<3>(lo), sbyte_f32<3>(hi));
-  }
-}
-
-}  // namespace
-
 // STAB: the block's whole [128 x G] fp16 group-scale table is loaded once, coalesced,
 // into LDS (G <= 128 and a multiple of 4, contiguous groups: at most 32 KiB).
 // Otherwise each stage loads the
@@ -219,8 +198,10 @@ __global__ __launch_bounds__(256, 2) void grouped_int4_kernel(const Mfma16Params
   };
   auto store_b = [&](auto r, const uint4& w, float t0, float t1) __attribute__((always_inline)) {
     uint4* bs = bbuf(r);
+    const uint32_t d[4] = {w.x, w.y, w.z, w.w};
     uint32_t o[16];
-    widen_int4x16<MT>(w, o);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) widen_int4x16<MT>(d[t], o + 4 * t);
 #pragma unroll
     for (int h = 0; h < 4; ++h)
       bs[b_row * 8 + ((4 * b_cc + h) ^ swz(b_row))] = make_uint4(o[4 * h + 0], o[4 * h + 1], o[4 * h + 2], o[4 * h + 3]);
@@ -542,31 +523,31 @@ int launch_grouped_partial(const Mfma16Params& p, hipStream_t st, bool bf16) {
   if (s < 1 || p.K % s != 0) return MLS_ERR_UNSUPPORTED;
   const int64_t kp = p.K / s, G = kp / p.group;
   if (kp % 64 != 0 || kp % p.group != 0) return MLS_ERR_UNSUPPORTED;
-  if (grouped_skinny_fits(p, false)) {
-    const int rc = launch_grouped_skinny(p, st, bf16, false, true);
-    if (rc != MLS_ERR_UNSUPPORTED) return rc;
-  }
   const int tmx = chunk_tmx(p.M, p.E);
   const bool stab = p.s_dt == MLS_F16 && p.ld_sg == 1 && G % 4 == 0 && G <= 32 && (p.ld_sn % 4) == 0 &&
                     (p.s_estride % 4) == 0 && aligned(p.s, 8);
+  if (grouped_skinny_fits(p)) {
+    const int rc = launch_grouped_skinny(p, st, bf16, false, true, stab);
+    if (rc != MLS_ERR_UNSUPPORTED) return rc;
+  }
   if (stab) return launch_partial_tmx<32>(p, st, bf16, tmx);
   if (p.s_dt == MLS_F16) return launch_partial_tmx<1>(p, st, bf16, tmx);
   return launch_partial_tmx<0>(p, st, bf16, tmx);
 }
 
 int launch_grouped_seg(const Mfma16Params& p, hipStream_t st, bool bf16, bool gate_up) {
-  Mfma16Params one = p;
-  one.ksplit = 1;
-  if (grouped_skinny_fits(one, gate_up)) {
-    const int rc = launch_grouped_skinny(one, st, bf16, gate_up, false);
-    if (rc != MLS_ERR_UNSUPPORTED) return rc;
-  }
   const int tmx = chunk_tmx(p.M, p.E);
   // scale table in LDS: fp16 scales, contiguous groups, G a multiple of 4 up to 128,
   // 8-byte aligned rows; a table of up to 32 groups keeps two blocks per CU
   const int64_t G = p.K / p.group;
   const bool stab = p.s_dt == MLS_F16 && p.ld_sg == 1 && G % 4 == 0 && G <= 128 && (p.ld_sn % 4) == 0 &&
                     (p.s_estride % 4) == 0 && aligned(p.s, 8) && (!gate_up || aligned(p.s2, 8));
+  Mfma16Params one = p;
+  one.ksplit = 1;
+  if (grouped_skinny_fits(one)) {
+    const int rc = launch_grouped_skinny(one, st, bf16, gate_up, false, stab);
+    if (rc != MLS_ERR_UNSUPPORTED) return rc;
+  }
   if (!stab && p.s_dt == MLS_F16)
     return gate_up ? launch_grouped_tmx<1, true>(p, st, bf16, tmx) : launch_grouped_tmx<1, false>(p, st, bf16, tmx);
   if (!stab)

@@ -159,6 +159,20 @@ __device__ __forceinline__ void widen_int4(const uint4& q, uint32_t* o) {
   }
 }
 
+// 8 INT4 weights (a dword, even k in the low nibble) -> 4 dwords of 16-bit floats holding 16 (v - 8)
+// in k order, exact, 16 VALU: the nibbles with their top bit flipped are two's complement, and in
+// the high half of a byte they convert as 16 (v - 8). The callers' fp32 results take the 1/16.
+template <typename MT>
+__device__ __forceinline__ void widen_int4x16(uint32_t d, uint32_t* o) {
+  const uint32_t x = d ^ 0x88888888u;
+  const uint32_t hi = x & 0xF0F0F0F0u;         // k = 1, 3, 5, 7 (byte b: k = 2b + 1)
+  const uint32_t lo = (x << 4) & 0xF0F0F0F0u;  // k = 0, 2, 4, 6
+  o[0] = pack_exact2<MT>(sbyte_f32<0>(lo), sbyte_f32<0>(hi));
+  o[1] = pack_exact2<MT>(sbyte_f32<1>(lo), sbyte_f32<1>(hi));
+  o[2] = pack_exact2<MT>(sbyte_f32<2>(lo), sbyte_f32<2>(hi));
+  o[3] = pack_exact2<MT>(sbyte_f32<3>(lo), sbyte_f32<3>(hi));
+}
+
 // 16 e4m3 bytes -> 16 bf16 (8 dwords, k order); exact: e4m3 is a subset of bf16.
 __device__ __forceinline__ void widen_e4m3(const uint4& q, uint32_t* o) {
   const uint32_t d[4] = {q.x, q.y, q.z, q.w};
@@ -210,9 +224,11 @@ int launch_grouped_seg(const Mfma16Params& p, hipStream_t st, bool bf16, bool ga
 // multiple of 64 and of the group and its scales fit the 32-group LDS table.
 int launch_grouped_partial(const Mfma16Params& p, hipStream_t st, bool bf16);
 // The grouped kernel for few rows an expert (grouped_skinny.hip); p.ksplit >= 1, partial: fp32
-// partial products of p.ksplit K ranges.
-bool grouped_skinny_fits(const Mfma16Params& p, bool gate_up);
-int launch_grouped_skinny(const Mfma16Params& p, hipStream_t st, bool bf16, bool gate_up, bool partial);
+// partial products of p.ksplit K ranges. Its results are the chunk kernel's bit for bit; table:
+// the chunk kernel would take its scale-table form.
+bool grouped_skinny_takes(int64_t M, int E, int64_t K, int group, int ksplit);
+bool grouped_skinny_fits(const Mfma16Params& p);
+int launch_grouped_skinny(const Mfma16Params& p, hipStream_t st, bool bf16, bool gate_up, bool partial, bool table);
 // K splits that give the down projection of an expert MLP (few column tiles) two
 // blocks per CU; 1 when no split is needed or possible.
 int grouped_splits(int64_t M, int E, int64_t N, int64_t K, int group);

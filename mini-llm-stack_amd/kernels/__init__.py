@@ -107,6 +107,7 @@ EXT_SIGNATURES = {
     "mlsx_int4_gemm": (SIGNATURES["mls_int4_gemm_ws"][0], _I),
     "mlsx_paged_attention_workspace": ([_I64, _I64, _I64, _I64, _I64], _I64),
     "mlsx_paged_attention_decode": (SIGNATURES["mls_paged_attention_decode"][0], _I),
+    "mlsx_int4_grouped_few_rows": ([_I64, _I, _I64, _I, _I], _I),
     "mlsx_route_topk": ([_P, _I, _I64, _I64, _I, _I, _P, _P, _P], _I),
     "mlsx_route_sort": ([_P, _I64, _I, _I, _P, _P, _P, _P, _P], _I),
     "mlsx_dw_fp32_workspace": ([_I64, _I64, _I64], _I64),

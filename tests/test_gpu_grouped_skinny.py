@@ -1,20 +1,20 @@
 """The grouped INT4 GEMMs for few rows an expert (csrc/grouped_skinny.hip) against float64.
 
-Bounds: a group's products are summed with an offset of 136 (bf16) or 1032 (fp16) a weight that
-is taken off afterwards, so an fp32 sum's error is that of terms up to 1032 |x| s: K 2^-24 of
-their root sum of squares covers it at these K; a 16-bit output rounds once (2^-8, 2^-11)."""
+Bounds: weights are exact, so an fp32 sum's error is that of K terms up to 8 |x| s: K 2^-24 of their
+root sum of squares covers it at these K; a 16-bit output rounds once (2^-8, 2^-11). And against
+the chunk kernel (csrc/gemm_grouped.hip), which takes calls of more rows: the same bits."""
 
 from __future__ import annotations
 
 import pytest
 import torch
 
+import kernels
 from kernels.moe_grouped import int4_grouped_gate_up, int4_grouped_matmul, int4_grouped_matmul_partial, segment_offsets
 
 pytestmark = pytest.mark.gpu
 
 ROUND = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
-OFF = {torch.bfloat16: 136.0, torch.float16: 1032.0}
 
 
 def _weights(dev, E, N, K, group, sdt, seed):
@@ -39,7 +39,7 @@ def _product(x, w, counts):
 
 
 def _slack(x, s, K):
-    return K * 2.0 ** -24 * OFF[x.dtype] * x.double().square().sum(1, keepdim=True).sqrt() * float(s.max())
+    return K * 2.0 ** -24 * 8.0 * x.double().square().sum(1, keepdim=True).sqrt() * float(s.max())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -78,3 +78,52 @@ def test_gate_up_with_gather(dev, counts, H, K, group, dtype):
     # |silu'| <= 1.1 and silu in fp32 with the device's exp: 2^-20 of the result
     bound = (ROUND[dtype] + 2.0 ** -20) * want.abs() + 1.1 * d * u.abs() + g.abs() * d + d * d
     assert float(((h.double() - want).abs() - bound).max()) <= 0
+
+
+def _takes(M, E, K, group, splits=1):
+    return kernels.lib().mlsx_int4_grouped_few_rows(M, E, K, group, splits) == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,N,K,group,sdt,splits", [
+    ([5, 0, 16, 2], 150, 384, 128, torch.float32, 3),    # an edge of columns, three steps
+    ([1, 9], 96, 2048, 64, torch.float16, 2), ([3, 1], 64, 896, 64, torch.float32, 1),
+    ([11, 14, 8, 15], 5632, 2048, 128, torch.float16, 4),   # two row tiles, blocks few and ranges long
+    ([9, 40, 0, 7, 12, 3, 13, 12], 3072, 2048, 128, torch.float16, 1), ([30, 1], 128, 2048, 512, torch.float32, 1),
+    ([2] * 8, 512, 2048, 256, torch.float16, 2), ([2, 2], 64, 14336, 64, torch.float32, 1),  # 224 groups' scales in LDS
+])
+def test_rows_are_the_chunk_kernels(dev, counts, N, K, group, sdt, splits, dtype):
+    """A row gets the same bits here and in a call of so many rows that the chunk kernel takes it,
+    with infinities and NaN among them: plain, in partial products, and gate/up."""
+    E, M = len(counts), sum(counts)
+    extra = 16 * E + 1  # more rows for expert 0, behind its own
+    assert _takes(M, E, K, group, splits) and not _takes(M + extra, E, K, group, splits)
+    (q, s, _), (qu, su, _) = (_weights(dev, E, N, K, group, sdt, K + i) for i in range(2))
+    x = _rows(dev, counts, K, dtype, N)
+    x[0, 3], x[M // 2, K - 1], x[M - 1, K // 2] = float("inf"), float("-inf"), float("nan")
+    big = torch.cat([x[:counts[0]], _rows(dev, [extra], K, dtype, 1), x[counts[0]:]])
+    few, many = torch.tensor(counts, device=dev), torch.tensor([counts[0] + extra, *counts[1:]], device=dev)
+
+    def same(a, b):
+        b = torch.cat([b[..., :counts[0], :], b[..., counts[0] + extra:, :]], -2)
+        bad = torch.isnan(a)
+        assert a.shape == b.shape and bad.any() and not bad.all()
+        assert torch.equal(bad, torch.isnan(b)) and torch.equal(a[~bad], b[~bad])
+
+    same(int4_grouped_matmul(x, q, s, few, group), int4_grouped_matmul(big, q, s, many, group))
+    same(int4_grouped_gate_up(x, q, s, qu, su, few, group), int4_grouped_gate_up(big, q, s, qu, su, many, group))
+    same(int4_grouped_matmul_partial(x, q, s, few, group, splits),
+         int4_grouped_matmul_partial(big, q, s, many, group, splits))
+
+
+def test_infinities_as_fp32(dev):
+    """fp32 scales (no scale table): an infinite x gives what fp32 arithmetic gives, +-inf, and NaN
+    only at weights of zero."""
+    q, s, w = _weights(dev, 2, 200, 512, 128, torch.float32, 1)
+    x = _rows(dev, [2, 3], 512, torch.bfloat16, 2)
+    x[1, 70], x[3, 511] = float("inf"), float("-inf")
+    y = int4_grouped_matmul(x, q, s, torch.tensor([2, 3], device=dev), 128).float()
+    want = torch.cat([x[:2].float() @ w[0].float().t(), x[2:].float() @ w[1].float().t()])
+    inf = torch.isinf(want)
+    assert inf.any() and torch.equal(y[inf], want[inf]) and torch.equal(torch.isnan(y), torch.isnan(want))
+    assert torch.isfinite(y[torch.isfinite(want)]).all()
