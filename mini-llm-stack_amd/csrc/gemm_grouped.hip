@@ -496,12 +496,7 @@ int grouped_splits(int64_t M, int E, int64_t N, int64_t K, int group) {
       if (tiles * s >= 512) break;  // two blocks per CU reached
     }
   }
-  if (env > 0) return 1;
-  // few rows an expert (grouped_skinny.hip): a block's wavefronts share a range, so ranges of at
-  // least 8 steps of 128 k (512 -> 128 k a wavefront: 11.1 us against 9.6 unsplit to that point)
-  if (M <= (int64_t)E * 8)
-    while (best > 2 && K / best < 1024) best /= 2;
-  return best;
+  return env > 0 ? 1 : best;
 }
 
 template <int SCL>

@@ -224,3 +224,14 @@ def test_paged_attention_rejects_and_sizes_workspace():
     assert call(st=16) == kernels.MLS_ERR_ARG                 # row stride below D
     assert call(btss=1) == kernels.MLS_ERR_ARG                # table rows overlap
     assert call(n=0) == 0
+
+
+@pytest.mark.parametrize("M,E,N,K,group,want", [
+    (32, 8, 2048, 2048, 32, 8), (32, 8, 2048, 1024, 32, 8), (64, 8, 1024, 5120, 32, 8), (64, 8, 1024, 7168, 32, 8),
+    (65, 8, 1024, 7168, 32, 8), (32, 8, 4096, 14336, 128, 4), (16, 4, 512, 1024, 64, 4),
+])
+def test_grouped_splits_of_a_decode_batch(M, E, N, K, group, want):
+    """Few rows an expert split K as more do: until there are two blocks a CU, by ranges of whole
+    64 k, whose groups are a multiple of 4 and at most the 32 of the kernels' scale table."""
+    s = kernels.load_library().mls_int4_grouped_splits(M, E, N, K, group)
+    assert s == want and K // s % 64 == 0 and K // s // group <= 32 and K // s // group % 4 == 0
