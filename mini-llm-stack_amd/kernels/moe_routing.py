@@ -77,6 +77,7 @@ class _Route:
         ints = torch.empty(n + n_experts + 1, dtype=torch.int32, device=dev)
         self.token_of_slot, self.seg_off = ints[:n], ints[n:]
         self.pos = torch.empty(idx.shape, dtype=torch.int64, device=dev)
+        # (the host allocator does not know of the launch that writes it: wait() before it goes)
         self.bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
         kernels.check(kernels.lib().mlsx_route_sort(
             idx.data_ptr(), n, idx.shape[1], n_experts, self.token_of_slot.data_ptr(), self.seg_off.data_ptr(),
@@ -85,8 +86,11 @@ class _Route:
         self.done.record(torch.cuda.current_stream(dev))
         self.n_experts = n_experts
 
-    def check(self) -> None:
+    def wait(self) -> None:
         self.done.synchronize()
+
+    def check(self) -> None:
+        self.wait()
         bad = int(self.bad)
         if bad == 2:
             raise RuntimeError("moe_dispatch_combine: negative expert index")
@@ -152,9 +156,13 @@ def moe_dispatch_combine(flat: torch.Tensor, weights: torch.Tensor, experts_idx:
     quantized = st is not None and flat.dtype in (torch.bfloat16, torch.float16)
     if quantized and _Route.takes(experts_idx, n_experts):
         route = _Route(experts_idx, n_experts)
-        out = int4_expert_mlp_combine(flat, route.seg_off, st["w_gate"][0], st["w_gate"][1], st["w_up"][0],
-                                      st["w_up"][1], st["w_down"][0], st["w_down"][1], st["group_size"], weights,
-                                      route.pos, a_rows=route.token_of_slot)
+        try:
+            out = int4_expert_mlp_combine(flat, route.seg_off, st["w_gate"][0], st["w_gate"][1], st["w_up"][0],
+                                          st["w_up"][1], st["w_down"][0], st["w_down"][1], st["group_size"], weights,
+                                          route.pos, a_rows=route.token_of_slot)
+        except BaseException:
+            route.wait()
+            raise
         route.check()
         return out
     token_of_slot, counts, pos = sort_by_expert(experts_idx, n_experts)
