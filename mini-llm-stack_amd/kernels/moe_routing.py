@@ -78,7 +78,7 @@ class _Route:
         self.token_of_slot, self.seg_off = ints[:n], ints[n:]
         self.pos = torch.empty(idx.shape, dtype=torch.int64, device=dev)
         # (the host allocator does not know of the launch that writes it: wait() before it goes)
-        self.bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self.bad = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)
         kernels.check(kernels.lib().mlsx_route_sort(
             idx.data_ptr(), n, idx.shape[1], n_experts, self.token_of_slot.data_ptr(), self.seg_off.data_ptr(),
             self.pos.data_ptr(), self.bad.data_ptr(), stream(dev)), "moe_dispatch_combine")

@@ -89,3 +89,11 @@ def test_combine_columns_over_blocks(dev, T, D):
     pos = torch.randperm(2 * T, generator=g).reshape(T, 2).to(dev)
     want = (x.double()[pos] * w.double()[:, :, None]).sum(1)
     assert float(((combine_rows(x, w, pos).double() - want).abs() - 2.0 ** -22 * (x.double()[pos].abs() * w[:, :, None]).sum(1)).max()) <= 0
+
+
+def test_sort_under_a_default_device(dev):
+    """The word that the kernel reports in is pinned host memory whatever torch's default device."""
+    with torch.device(dev):
+        r = _Route(torch.tensor([[1, 0], [2, 2]]), 3)
+    r.check()
+    assert r.bad.device.type == "cpu" and r.bad.is_pinned() and r.seg_off.tolist() == [0, 1, 2, 4]
