@@ -4,6 +4,9 @@ strides and the HIP stream of the calling thread."""
 from __future__ import annotations
 
 import torch
+from torch import _C, _ops
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from kernels import MLS_BF16, MLS_F16, MLS_F32
 
@@ -62,9 +65,18 @@ def scale_vector(scale: torch.Tensor) -> tuple[torch.Tensor, int]:
     return scale, _DT[scale.dtype]
 
 
+def _watched() -> bool:
+    """Whether something records, rewrites or intercepts this thread's torch calls: a trace, a function
+    transform, forward mode, a dispatch mode, or a function mode other than torch's default device."""
+    return (_C._is_tracing() or _C._len_torch_dispatch_stack() > 0 or forward_ad._current_level >= 0
+            or _C._functorch.peek_interpreter_stack() is not None or _ops._len_torch_dispatch_stack_pre_dispatch() > 0
+            or torch.compiler.is_compiling()
+            or _C._len_torch_function_stack() > 0
+            and not all(isinstance(m, DeviceContext) for m in torch.overrides._get_current_function_mode_stack()))
+
+
 def plain(t: torch.Tensor) -> bool:
-    """An ordinary device tensor outside tracing and function transforms, from which no gradient
-    is asked for: one whose memory a kernel may read in place of differentiable torch ops."""
+    """An ordinary device tensor whose values are as stored, from which no gradient is asked for, in
+    code that nothing watches: one whose memory a kernel may read in place of torch ops."""
     return (type(t) is torch.Tensor and t.device.type == "cuda" and not (t.requires_grad and torch.is_grad_enabled())
-            and not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0)
+            and not t.is_neg() and not _watched())

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import kernels
+from kernels._hip import plain
 from kernels.moe_routing import _Route, combine_rows, route_topk, sort_by_expert
 
 pytestmark = pytest.mark.gpu
@@ -54,6 +55,40 @@ def test_topk_keeps_gradients(dev):
     _, t = torch.func.jvp(lambda v: route_topk(v, 2)[0], (x.detach(),), (torch.ones_like(x),))
     assert t.shape == (6, 2)
     assert torch.vmap(lambda v: route_topk(v, 2)[0])(x.detach().reshape(2, 3, 8)).shape == (2, 3, 2)
+
+
+def test_traces_and_modes_see_the_torch_ops(dev):
+    """Under a trace the result depends on the traced input (a kernel's would be a constant), and
+    dispatch and function modes see topk; torch's default device alone changes nothing."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    a, b = (torch.randn(4, 8, generator=torch.Generator().manual_seed(i)).to(dev) for i in range(2))
+    want = route_topk(b, 2)
+    for traced in (torch.jit.trace(lambda t: route_topk(t, 2), a), make_fx(lambda t: route_topk(t, 2))(a),
+                   make_fx(lambda t: route_topk(t, 2), pre_dispatch=True)(a)):
+        w, e = traced(b)
+        assert torch.equal(e, want[1]) and torch.allclose(w, want[0])
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Dispatch, Function):
+        seen.clear()
+        with mode():
+            route_topk(a, 2)
+        assert any("topk" in n for n in seen), seen
+    with torch.device(dev):
+        assert plain(a) and _Route.takes(want[1], 8)
 
 
 @pytest.mark.parametrize("T,k,E", [(1, 1, 1), (1, 2, 8), (37, 2, 3), (512, 2, 8), (1025, 1, 256), (4096, 8, 64)])
