@@ -31,8 +31,9 @@ int mlsx_int4_gemm(const void* a, int a_dt, int64_t lda, const uint8_t* w, int64
 /* ---------------------------------------------------------------- paged attention */
 
 /* mls_paged_attention_decode with the contexts cut into pieces of equal length instead of as
- * many splits a sequence, so that a batch of unequal lengths keeps the GPU even. Arguments as
- * there; the workspace holds mlsx_paged_attention_workspace floats (0: none). */
+ * many splits a sequence, so that a batch of unequal lengths keeps the GPU even; the length comes
+ * from the batch's contexts, on the device, whatever the tables' width. Arguments as there; the
+ * workspace holds mlsx_paged_attention_workspace floats (0: none). */
 int64_t mlsx_paged_attention_workspace(int64_t n_seqs, int64_t H, int64_t D, int64_t block_size, int64_t max_blocks);
 int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss, int64_t q_sh, const void* k_pool,
                                 const void* v_pool, int kv_dt, int64_t kv_sb, int64_t kv_sh, int64_t kv_st,

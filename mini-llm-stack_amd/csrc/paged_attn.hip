@@ -23,6 +23,7 @@
 // [0, num_blocks) is skipped (its tokens weigh 0) rather than dereferenced, and a
 // context longer than the table row covers is cut at the row's end. A zero context
 // gives a zero output, as in the reference.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -82,7 +83,11 @@ struct PagedArgs {
   float scale;
   float* ws;  // splits > 1: [n_seqs][H][splits][D + 2] (acc[D], m, l)
   int splits;
-  int per;  // least table blocks of a piece (piece_blocks); 0: a sequence's blocks over `splits`
+  // least table blocks of a piece (piece_blocks); 0: a sequence's blocks over `splits`
+  int per;
+  // batches past 256 sequences: pieces of at most `cap` blocks, and at least `share` of them where
+  // a sequence has the blocks
+  int cap, share;
 };
 
 // Table blocks of a sequence's cached tokens, never past its table row.
@@ -90,22 +95,33 @@ __device__ __forceinline__ int live_blocks(const PagedArgs& a, int ctx) {
   return (int)min((int64_t)((max(ctx, 0) + a.BS - 1) / a.BS), a.max_blocks);
 }
 
-// Table blocks a piece, where contexts are cut into pieces of one length (a.per > 0): the length
-// that makes about 4096 pieces of the batch's own blocks, a.per (from the largest context the
-// tables allow) at least. Every wavefront of both kernels finds the same value: one load of
-// the lengths and a sum. Batches past 256 sequences take a.per.
+// Table blocks a piece of a sequence of nb blocks, where contexts are cut into pieces of one length
+// (a.per > 0): the length that makes about 4096 pieces of the batch's own blocks, and at most
+// a.splits of the longest context, a.per at least. Every wavefront of both kernels finds the same
+// value: one load of the lengths, a sum and a maximum. The width of the tables only bounds a.splits,
+// the wavefronts that a sequence and head can have (pieces sized by it: one context of 4096, 32
+// heads, a table for 131072 tokens, 98 us; 21 so, 29 in even shares of the context).
+// Batches past 256 sequences have the wavefronts without a cut: a.share pieces of a sequence's own
+// blocks, or more where those would be longer than a.cap.
 // (32 heads of 128, bf16, us: 40 sequences of 1 to 4096 tokens 98 as 4 splits a sequence, which
 // wait for the longest one's, 80 as pieces; 64 of 1 to 2048 tokens 92 and 70; all 2048 long 331
 // and 328. Eight heads, one sequence of 4096: 38 and 20, mostly the table's register.)
-__device__ __forceinline__ int piece_blocks(const PagedArgs& a, int lane) {
-  if (a.n_seqs > 256) return a.per;
-  int sum = 0;
+__device__ __forceinline__ int piece_blocks(const PagedArgs& a, int lane, int nb) {
+  if (a.n_seqs > 256) return max(min((nb + a.share - 1) / a.share, a.cap), a.per);
+  int sum = 0, most = 0;
   for (int s0 = 0; s0 < a.n_seqs; s0 += 64)
-    if (s0 + lane < a.n_seqs) sum += live_blocks(a, a.ctx[s0 + lane]);
+    if (s0 + lane < a.n_seqs) {
+      const int n = live_blocks(a, a.ctx[s0 + lane]);
+      sum += n;
+      most = max(most, n);
+    }
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  for (int off = 32; off >= 1; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+    most = max(most, __shfl_xor(most, off, 64));
+  }
   const int want = (int)min(((int64_t)sum * a.H + 4095) / 4096, (int64_t)0x3FFFFFFF);
-  return __builtin_amdgcn_readfirstlane(max(want, a.per));
+  return __builtin_amdgcn_readfirstlane(max(max(want, (most + a.splits - 1) / a.splits), a.per));
 }
 
 // Table blocks [b0, b1) of split `split` of a sequence of nb blocks, and how many of its splits
@@ -118,7 +134,7 @@ __device__ __forceinline__ int split_range(const PagedArgs& a, int nb, int split
     b1 = min(nb, b0 + per);
     return a.splits;
   }
-  const int live = max((nb + piece - 1) / piece, 1), per = (nb + live - 1) / live;
+  const int live = min(max((nb + piece - 1) / piece, 1), a.splits), per = (nb + live - 1) / live;
   b0 = min(split * per, nb);  // (split < a.splits, so the product stays below twice the table)
   b1 = min(nb, b0 + per);
   return live;
@@ -162,7 +178,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const PagedArgs a) {
   const int ctx = a.ctx[seq];
   const int nb = live_blocks(a, ctx);
   int b0, b1;
-  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane, nb) : 0, b0, b1);
   if (split >= live) return;
   float q[EPC];
   {
@@ -309,7 +325,7 @@ __global__ __launch_bounds__(256) void paged_attn_generic_kernel(const PagedArgs
   const int ctx = a.ctx[seq];
   const int nb = live_blocks(a, ctx);
   int b0, b1;
-  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  const int live = split_range(a, nb, split, a.per > 0 ? piece_blocks(a, lane, nb) : 0, b0, b1);
   if (split >= live) return;
   float m = NEG_INF, l = 0.0f;
   const int32_t* table = a.bt + (int64_t)seq * a.bt_ss;
@@ -363,7 +379,7 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(const PagedArgs a
   const int head = (int)(item % a.H), seq = __builtin_amdgcn_readfirstlane((int)(item / a.H));
   const int nb = live_blocks(a, a.ctx[seq]);
   int b0, b1;
-  const int live = split_range(a, nb, 0, a.per > 0 ? piece_blocks(a, lane) : 0, b0, b1);
+  const int live = split_range(a, nb, 0, a.per > 0 ? piece_blocks(a, lane, nb) : 0, b0, b1);
   if (live == 1) return;  // written by its only split
   const float* w = a.ws + item * a.splits * (a.D + 2);
   const float ms = lane < live ? w[lane * (a.D + 2) + a.D] : NEG_INF;
@@ -400,17 +416,29 @@ int choose_splits(int64_t n_seqs, int64_t H, int64_t max_blocks) {
   return (int)(s < 64 ? s : 64);
 }
 
-// The least piece length, in table blocks: 128 tokens, or more where that would make over 16384
-// wavefronts or 64 splits a sequence. (64 and 256 tokens against 128, us: 4 sequences of up to
-// 1000 tokens, 32 heads, 19.5 and 18.3 against 13.7; one of 4096, 8 heads, 37 and 25 against 26.)
-int choose_per(int64_t n_seqs, int64_t H, int64_t block_size, int64_t max_blocks) {
-  const int64_t tokens = max_blocks * block_size, items = n_seqs * H;
-  int64_t piece = cdiv(items * tokens, 16384);
-  piece = piece > 128 ? piece : 128;
-  int64_t per = cdiv(piece, block_size);
-  const int64_t least = cdiv(max_blocks, 64);
-  per = per > least ? per : least;
-  return (int)(per < 0x3FFFFFFF ? per : 0x3FFFFFFF);
+// How contexts are cut (a.per, a.cap, a.share, a.splits), from the sizes that the host knows. Pieces
+// have 128 tokens at least. (64 and 256 tokens against 128, us: 4 sequences of up to 1000 tokens,
+// 32 heads, 19.5 and 18.3 against 13.7; one of 4096, 8 heads, 37 and 25 against 26.) The grid has room for
+// 64 pieces a sequence, less where the tables are shorter or that would be over about 16384
+// wavefronts. Past 256 sequences, whose lengths the kernels don't sum: as many even pieces as
+// choose_splits gives, none longer than a full table's blocks make 16384 wavefronts of (300
+// sequences of 1 to 2048 tokens, 8 heads, 98 us in 2 even shares, 75 so; 32 heads 309 uncut, 265 so).
+// Where sequences and heads alone are the 4096 wavefronts that choose_splits aims at, no context
+// under 1024 tokens is cut (300 of 700 tokens, 32 heads, 550 us in two pieces, 518 in one).
+void choose_pieces(PagedArgs& a, int64_t n_seqs, int64_t H, int64_t block_size, int64_t max_blocks) {
+  const int64_t pairs = n_seqs * H, least = cdiv(128, block_size);
+  const int64_t room = std::min<int64_t>(64, std::max<int64_t>(cdiv(16384, pairs), 1));
+  int64_t splits = std::max<int64_t>(std::min(cdiv(max_blocks, least), room), 1), cap = cdiv(max_blocks, splits);
+  const int share = choose_splits(n_seqs, H, max_blocks);
+  if (n_seqs > 256) {
+    const int64_t tokens = std::max<int64_t>(cdiv(pairs * max_blocks * block_size, 16384), pairs >= 4096 ? 1024 : 128);
+    cap = std::max(cdiv(tokens, block_size), cdiv(max_blocks, 64));
+    splits = std::max<int64_t>(cdiv(max_blocks, cap), std::min<int64_t>(share, cdiv(max_blocks, least)));
+  }
+  a.per = (int)least;
+  a.cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), 0x3FFFFFFF);
+  a.share = share;
+  a.splits = (int)splits;
 }
 
 template <typename QT, typename KT>
@@ -493,7 +521,7 @@ int paged_prepare(const char* fn, const void* q, int q_dt, int64_t q_ss, int64_t
   if (!fast && D > 256) return fail(MLS_ERR_UNSUPPORTED, "%s: head dim %lld needs 16-byte rows", fn, (long long)D);
   a = PagedArgs{q, q_ss, q_sh, k_pool, v_pool, kv_sb, kv_sh, kv_st, num_blocks, block_tables, bt_ss,
                 max_blocks, context_lens, out, o_ss, o_sh, (int)n_seqs, (int)H, (int)D, (int)block_size,
-                scale, nullptr, splits, 0};
+                scale, nullptr, splits, 0, 0, 0};
   return MLS_OK;
 }
 
@@ -531,8 +559,9 @@ extern "C" int mls_paged_attention_decode(const void* q, int q_dt, int64_t q_ss,
 extern "C" int64_t mlsx_paged_attention_workspace(int64_t n_seqs, int64_t H, int64_t D, int64_t block_size,
                                                   int64_t max_blocks) {
   if (n_seqs <= 0 || H <= 0 || D <= 0 || block_size <= 0 || max_blocks <= 0) return 0;
-  const int64_t s = cdiv(max_blocks, choose_per(n_seqs, H, block_size, max_blocks));
-  return s > 1 ? n_seqs * H * s * (D + 2) : 0;
+  PagedArgs a{};
+  choose_pieces(a, n_seqs, H, block_size, max_blocks);
+  return a.splits > 1 ? n_seqs * H * a.splits * (D + 2) : 0;
 }
 
 extern "C" int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss, int64_t q_sh,
@@ -552,10 +581,7 @@ extern "C" int mlsx_paged_attention_decode(const void* q, int q_dt, int64_t q_ss
                          scale, a, need, fast, cpt, done);
   if (rc != MLS_OK || done) return rc;
   a.splits = 1;
-  if (max_blocks > 0) {
-    a.per = choose_per(n_seqs, H, block_size, max_blocks);
-    a.splits = (int)cdiv(max_blocks, a.per);
-  }
+  if (max_blocks > 0) choose_pieces(a, n_seqs, H, block_size, max_blocks);
   need = a.splits > 1 ? n_seqs * H * a.splits * (D + 2) : 0;
   if (need > 0 && (!workspace || workspace_floats < need))
     return fail(MLS_ERR_ARG, "%s: workspace of %lld floats needed (mlsx_paged_attention_workspace)", fn,

@@ -31,6 +31,8 @@ def _want(q, k, v, tab, lens, bs):
     ([5000, 5000], 1, 8, 0), ([1024 + 1], 2, 1, 0),   # more than 64 blocks a piece
     ([40] * 300 + [2000], 2, 32, 0),         # past 256 sequences: the length from the table's width
     ([2048] * 3, 32, 16, -20),               # contexts past the table's end are cut there
+    ([500, 3, 129], 4, 16, 1000),            # a table 32 times as wide as the longest context
+    ([40] * 299 + [900, 2000], 8, 16, 4000), ([300] * 260, 16, 16, 600),
 ])
 def test_pieces(dev, lens, H, bs, extra, dtype, D):
     g = torch.Generator().manual_seed(len(lens) + max(lens))
@@ -51,9 +53,27 @@ def test_pieces(dev, lens, H, bs, extra, dtype, D):
     assert float(((y.double() - want).abs() - bound).max()) <= 0
 
 
+@pytest.mark.parametrize("lens,H", [([4096], 8), ([4096] * 8, 4), ([700, 1, 90], 4), ([200] * 300, 2)])
+def test_pieces_do_not_depend_on_the_tables_width(dev, lens, H):
+    """The contexts alone say how they are cut: a table 32 times as wide gives the same bits (a cut
+    at other tokens would round differently), so it is walked by as many wavefronts."""
+    bs, D, n = 16, 64, len(lens)
+    g = torch.Generator().manual_seed(n)
+    need = -(-max(lens) // bs)
+    k, v = (torch.randn(64, H, bs, D, generator=g).bfloat16().to(dev) for _ in range(2))
+    q = torch.randn(n, H, D, generator=g).bfloat16().to(dev)
+    wide = torch.randint(0, 64, (n, 32 * need), generator=g, dtype=torch.int32).to(dev)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=dev)
+    # (a table at least 64 pieces wide: the grid's room for pieces is the same in both)
+    mid = max(need, 64 * 128 // bs)
+    assert torch.equal(paged_attention_decode(q, k, v, wide[:, :mid], ctx), paged_attention_decode(q, k, v, wide, ctx))
+
+
 def test_workspace_sizes():
     L = kernels.lib()
     assert L.mlsx_paged_attention_workspace(4, 8, 64, 16, 8) == 0                  # one piece
     assert L.mlsx_paged_attention_workspace(4, 8, 64, 16, 9) == 4 * 8 * 2 * 66
     assert L.mlsx_paged_attention_workspace(1, 1, 64, 16, 1 << 20) == 64 * 66      # at most 64 splits
     assert L.mlsx_paged_attention_workspace(0, 8, 64, 16, 9) == 0
+    assert L.mlsx_paged_attention_workspace(40, 32, 128, 16, 1 << 16) == 40 * 32 * 13 * 130  # about 16384 wavefronts
+    assert L.mlsx_paged_attention_workspace(300, 32, 128, 16, 44) == 0             # enough wavefronts uncut
