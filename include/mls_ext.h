@@ -20,6 +20,9 @@ extern "C" {
  * aligned; 0: none): shapes whose tiles would not fill the GPU, or whose K is a multiple of
  * 32 but not of 64, run with the reduction axis split over blocks and fp32 partial products
  * in the workspace (gemm_ksplit.hip); every other call is the _ws one. */
+/* The number of ranges that K is split into for such a call, 1: these kernels unsplit, 0: the _ws entry
+ * point's kernels (faster there by the models of both). */
+int mlsx_wq_ksplit(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group);
 int64_t mlsx_wq_workspace(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group);
 int mlsx_int8_gemm(const void* a, int a_dt, int64_t lda, const int8_t* w, int64_t ldw, const void* s, int s_dt,
                    void* c, int c_dt, int64_t ldc, int64_t M, int64_t N, int64_t K, void* workspace,

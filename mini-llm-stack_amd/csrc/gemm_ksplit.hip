@@ -524,8 +524,8 @@ KsPlan best_tile(int wbits, int64_t M, int64_t N, int64_t K, int group, int part
   return best;
 }
 
-// What the general entry points would take for a shape, in us (infinity: the kernel with one
-// thread an output; 0: always theirs).
+// What the general entry points would take for a shape, in us (0: always theirs; infinity: the kernel
+// with one thread an output).
 float general_us(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group, bool split) {
   const bool f32 = a_dt == MLS_F32;
   const int ks = wbits == 4 && group % 128 == 0 ? 128 : 64;  // k a step of the skinny and medium kernels
@@ -534,9 +534,9 @@ float general_us(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group
     const int64_t m = split ? split_rows(M) : M, bm = split && wbits == 8 && m >= 256 ? 256 : 128;
     if ((split ? m <= 512 : M <= 256) && cdiv(m, bm) * cdiv(N, 256) < 128)
       return small_estimate_us(wbits, m, N, K, group, f32 ? 4 : 2, split);
-    return 1e30f;
+    return engine_estimate_us(wbits, m, N, K, group, split);
   }
-  if (M > 16 && !f32 && K % 64 == 0) return 1e30f;  // the engine
+  if (M > 16 && !f32 && K % 64 == 0) return engine_estimate_us(wbits, M, N, K, group, false);
   if (M > 1 && M <= 16 && stepped) return 0.0f;     // the skinny MFMA kernel
   // the register GEMVs: a pass over the weights for every `rows` rows of x (their registers
   // hold rows * K / 64 values a lane); measured 0.2 us a pass plus 0.15
@@ -565,7 +565,8 @@ KsPlan ks_plan(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) 
   if (general == 0.0f) return {};
   float us;
   const KsPlan p = best_tile(wbits, M, N, K, group, !f32 ? 1 : split ? 2 : 3, &us);
-  if (p.bm == 0 || us >= 0.92f * general) return {};  // (both models are off by a tenth or so)
+  if (f32) us += split_estimate_us(M, K);
+  if (p.bm == 0 || us >= general) return {};
   // whole 192- or 256-column tiles without a split are the engine's own
   if (p.splits == 1 && p.bn > 128 && K % 64 == 0) return {};
   return p;
@@ -594,6 +595,12 @@ extern "C" int64_t mlsx_wq_workspace(int wbits, int64_t M, int64_t N, int64_t K,
   const KsPlan pl = ks_plan(wbits, M, N, K, a_dt, group);
   const int64_t need = pl.bm ? ws_need(pl, M, N, K) : 0;
   return need > base ? need : base;
+}
+
+extern "C" int mlsx_wq_ksplit(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) {
+  if ((wbits != 4 && wbits != 8) || M <= 0 || N <= 0 || K <= 0 || !is_float_dt(a_dt)) return 0;
+  const KsPlan pl = ks_plan(wbits, M, N, K, a_dt, group);
+  return pl.bm ? pl.splits : 0;
 }
 
 extern "C" int mlsx_int8_gemm(const void* a, int a_dt, int64_t lda, const int8_t* w, int64_t ldw, const void* s,

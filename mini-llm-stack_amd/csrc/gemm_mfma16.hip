@@ -959,9 +959,9 @@ __global__ __launch_bounds__(64 * WM * WN) void mfma16_w4_kernel(const Mfma16Par
 
 // Whether mfma16_w4_kernel takes a dense INT4 GEMM: its coefficient table holds the groups
 // (group a multiple of 32, G <= kW4MaxGroups); MLS_W4 = 0 keeps the 128-row kernel (A/B runs).
-static bool w4_ok(const Mfma16Params& p) {
+static bool w4_ok(int64_t M, int64_t K, int group) {
   static const bool on = env_int("MLS_W4", 1) != 0;
-  return on && p.group % 32 == 0 && p.K % p.group == 0 && p.K / p.group <= kW4MaxGroups && p.M >= 256;
+  return on && group % 32 == 0 && K % group == 0 && K / group <= kW4MaxGroups && M >= 256;
 }
 
 template <typename MT, typename OT, bool SPLIT = false>
@@ -1042,6 +1042,19 @@ static int pick_bm(int64_t M, int64_t N, int max_bm) {
   return best;
 }
 
+// INT4: 256 x 128 tiles when they take no more rounds of 256 blocks than 128 x 256 tiles.
+static bool w4_rounds(int64_t M, int64_t N) {
+  return cdiv(cdiv(M, 256) * cdiv(N, 128), 256) <= cdiv(cdiv(M, 128) * cdiv(N, 256), 256);
+}
+
+// INT8 on 256-row tiles: 192 columns when fewer rounds of 256 blocks outweigh the smaller tile:
+// e.g. 2048 x 11008 is 344 blocks of 256 x 256 (two rounds, the second a third full) but 464
+// blocks of 256 x 192 (two rounds, 25% less work each); else 256.
+static int w8_columns(int64_t M, int64_t N) {
+  const int64_t mt = cdiv(M, 256);
+  return cdiv(mt * cdiv(N, 192), 256) * 192 < cdiv(mt * cdiv(N, 256), 256) * 256 ? 192 : 256;
+}
+
 // Tuning overrides for sweeps: MLS_BYTES = 0 keeps 256-row exact fp8 tiles on the kernel here
 // instead of the byte-operand kernel (gemm_bytes.hip), MLS_MFMA_WAVES = 4 or 8 wavefronts per block (default 8:
 // two per SIMD, so one wavefront's memory waits overlap the other's MFMAs), MLS_MFMA_BM =
@@ -1066,23 +1079,14 @@ static int dense16(Mfma16Params p, hipStream_t st) {
                               __is_same(OT, float) ? MLS_F32 : __is_same(OT, _Float16) ? MLS_F16 : MLS_BF16);
   }
   if constexpr (AKIND == A_RAW16 && BKIND == B_INT4) {
-    // 256 x 128 tiles on the INT4 kernel with the INT8 kernel's schedule, when they take no
-    // more rounds of 256 blocks than the 128 x 256 tiles
-    if (adma && w8 && w4_ok(p)) {
-      const int64_t b_w4 = cdiv(p.M, 256) * cdiv(p.N, 128), b_128 = cdiv(p.M, 128) * cdiv(p.N, 256);
-      if (cdiv(b_w4, 256) <= cdiv(b_128, 256)) return launch_w4<MT, OT>(p, st);
-    }
+    // 256 x 128 tiles on the INT4 kernel with the INT8 kernel's schedule
+    if (adma && w8 && w4_ok(p.M, p.K, p.group) && w4_rounds(p.M, p.N)) return launch_w4<MT, OT>(p, st);
   }
   if constexpr (AKIND == A_RAW16) {
     if (adma && w8 && bm == 256) {
       if constexpr (MAXBM >= 256) {
-        // 256 x 192 tiles when fewer rounds of 256 blocks outweigh the smaller tile:
-        // e.g. 2048 x 11008 is 344 blocks of 256 x 256 (two rounds, the second a
-        // third full) but 464 blocks of 256 x 192 (two rounds, 25% less work each)
         static const int force_bn = env_int("MLS_MFMA_BN", 0);
-        const int64_t mt = cdiv(p.M, 256);
-        const int64_t c256 = cdiv(mt * cdiv(p.N, 256), 256) * 256, c192 = cdiv(mt * cdiv(p.N, 192), 256) * 192;
-        if (force_bn == 192 || (force_bn != 256 && c192 < c256))
+        if (force_bn == 192 || (force_bn != 256 && w8_columns(p.M, p.N) == 192))
           return launch_adma<BKIND, MT, OT, 256, 192, 2, 4, false>(p, st);
         return launch_adma<BKIND, MT, OT, 256, 256, 2, 4, false>(p, st);
       }
@@ -1148,16 +1152,36 @@ int launch_gemm_wq_mfma_split(int wbits, const WqArgs& w, int64_t m_out) {
   p.m_out = (int)m_out;
   if (wbits == 8 && w.M >= 256) {
     p.m_tiles = (int)cdiv(p.M, 256);
-    const int64_t mt = p.m_tiles;
-    const int64_t c256 = cdiv(mt * cdiv(p.N, 256), 256) * 256, c192 = cdiv(mt * cdiv(p.N, 192), 256) * 192;
-    if (c192 < c256) return launch_adma<B_INT8, __bf16, float, 256, 192, 2, 4, false, true>(p, w.stream);
+    if (w8_columns(p.M, p.N) == 192) return launch_adma<B_INT8, __bf16, float, 256, 192, 2, 4, false, true>(p, w.stream);
     return launch_adma<B_INT8, __bf16, float, 256, 256, 2, 4, false, true>(p, w.stream);
   }
-  if (wbits == 4 && w4_ok(p) && cdiv(cdiv(p.M, 256) * cdiv(p.N, 128), 256) <= cdiv(cdiv(p.M, 128) * cdiv(p.N, 256), 256))
-    return launch_w4<__bf16, float, true>(p, w.stream);
+  if (wbits == 4 && w4_ok(p.M, p.K, p.group) && w4_rounds(p.M, p.N)) return launch_w4<__bf16, float, true>(p, w.stream);
   p.m_tiles = (int)cdiv(p.M, 128);
   if (wbits == 8) return launch_adma<B_INT8, __bf16, float, 128, 256, 2, 4, false, true>(p, w.stream);
   return launch_adma<B_INT4, __bf16, float, 128, 256, 2, 4, false, true>(p, w.stream);
+}
+
+// us of the engine for M rows (split rows: of the split matrix): rounds of 256 blocks, each walking
+// K / 64 stages of the tile's own time. Fitted to 640 timed shapes of 48 to 8192 rows (512 x 2048 to
+// 8192 x 8192 and 4096 x 11008, INT8 and INT4 with groups of 32, 64 and 128; error 1 to 6% rms).
+float engine_estimate_us(int wbits, int64_t M, int64_t N, int64_t K, int group, bool split) {
+  const float stages = (float)cdiv(K, 64), pass = split ? split_estimate_us(M / 2, K) : 0.0f;
+  auto us = [&](int bm, int bn, float stage, float edge) {
+    return pass + (float)cdiv(cdiv(M, bm) * cdiv(N, bn), 256) * (stages * stage + edge);
+  };
+  const int bm = split ? (wbits == 8 && M >= 256 ? 256 : 128) : pick_bm(M, N, wbits == 4 ? 128 : 256);
+  if (wbits == 8) {
+    if (bm == 256) return w8_columns(M, N) == 192 ? us(256, 192, 1.074f, 13.6f) : us(256, 256, 1.462f, 13.3f);
+    return bm == 128 ? us(128, 256, 0.939f, 11.3f) : bm == 64 ? us(64, 256, 1.038f, 6.8f)
+           : bm == 32 ? us(32, 256, 0.959f, 1.2f) : us(16, 256, 0.739f, 2.9f);
+  }
+  const int g = group >= 128 ? 2 : group == 64 ? 1 : 0;
+  static constexpr float w4[3] = {1.562f, 1.222f, 1.078f}, t128[3] = {1.918f, 1.566f, 1.515f},
+                         t64[3] = {2.594f, 2.25f, 2.067f}, t32[3] = {2.07f, 1.86f, 1.74f},
+                         t16[3] = {1.862f, 1.724f, 1.72f};
+  if (w4_ok(M, K, group) && w4_rounds(M, N)) return us(256, 128, w4[g], 6.7f);
+  return bm == 128 ? us(128, 256, t128[g], 7.0f) : bm == 64 ? us(64, 256, t64[g], 7.0f)
+         : bm == 32 ? us(32, 256, t32[g], 3.0f) : us(16, 256, t16[g], 0.0f);
 }
 
 int launch_grouped_int4(const GroupedArgs& g) {

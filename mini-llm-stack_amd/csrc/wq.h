@@ -46,6 +46,9 @@ float small_estimate_us(int wbits, int64_t M, int64_t N, int64_t K, int group, i
 
 // MFMA tiled GEMM for 16-bit activations. MLS_ERR_UNSUPPORTED outside its fast path.
 int launch_gemm_wq_mfma(int wbits, const WqArgs& p);
+// Its time for a shape in us, by a fitted model (split: M counts the rows of the split matrix, and
+// the pass that splits x is added).
+float engine_estimate_us(int wbits, int64_t M, int64_t N, int64_t K, int group, bool split);
 
 // Any shape, any dtype: one thread per output element.
 int launch_gemm_wq_generic(int wbits, const WqArgs& p);
@@ -60,6 +63,8 @@ int launch_gemv_mfma_split(int wbits, const WqArgs& p);
 int launch_gemm_wq_mfma_split(int wbits, const WqArgs& p, int64_t m_out);
 // x fp32 [M][ldx] -> split rows [split_rows(M)][K] bf16 (zeros for rows past M).
 int launch_split_rows(const float* x, int64_t ldx, int64_t M, int64_t K, void* x2, hipStream_t st);
+// Its time in us: 1.7 plus 2.0 a million values (fitted to 270 timed fp32 calls, 48 to 4096 rows).
+inline float split_estimate_us(int64_t M, int64_t K) { return 1.7f + 2.0e-6f * (float)M * (float)K; }
 // x fp32 [M][ldx] -> `parts` (2 or 3) bf16 rows per row, row m's part t at row
 // 16 parts (m / 16) + 16 t + m % 16 of x2 [16 parts ceil(M / 16)][K] (zeros past M): hi + lo
 // (x to 2^-16), or three parts that add up to x exactly.

@@ -103,6 +103,7 @@ ROUTE_MAX = 32768  # MLSX_ROUTE_MAX
 ROUTE_MAX_EXPERTS, ROUTE_MAX_TOP = 256, 8
 EXT_SIGNATURES = {
     "mlsx_wq_workspace": ([_I, _I64, _I64, _I64, _I, _I], _I64),
+    "mlsx_wq_ksplit": ([_I, _I64, _I64, _I64, _I, _I], _I),
     "mlsx_int8_gemm": (SIGNATURES["mls_int8_gemm_ws"][0], _I),
     "mlsx_int4_gemm": (SIGNATURES["mls_int4_gemm_ws"][0], _I),
     "mlsx_paged_attention_workspace": ([_I64, _I64, _I64, _I64, _I64], _I64),

@@ -235,3 +235,15 @@ def test_grouped_splits_of_a_decode_batch(M, E, N, K, group, want):
     64 k, whose groups are a multiple of 4 and at most the 32 of the kernels' scale table."""
     s = kernels.load_library().mls_int4_grouped_splits(M, E, N, K, group)
     assert s == want and K // s % 64 == 0 and K // s // group <= 32 and K // s // group % 4 == 0
+
+
+@pytest.mark.parametrize("bits,M,N,K,group,taken", [
+    (8, 1500, 5632, 5632, 0, False), (8, 2048, 5632, 2048, 0, False), (8, 700, 11008, 2048, 0, False),
+    (8, 2048, 11008, 4096, 0, False),                                 # whole 192-column tiles: the engine's own
+    (8, 333, 4096, 11008, 0, True), (4, 333, 4096, 11008, 128, True), (4, 16384, 4096, 4096, 128, True),
+    (4, 1, 4096, 4096, 128, False), (8, 12, 4096, 4096, 0, False),
+])
+def test_the_k_split_gemm_takes_what_it_is_faster_at(bits, M, N, K, group, taken):
+    """The plan is compared with the time of the kernel that would otherwise serve the shape, the
+    engine's among them (bf16)."""
+    assert (kernels.load_library().mlsx_wq_ksplit(bits, M, N, K, kernels.MLS_BF16, group) > 0) == taken
