@@ -19,7 +19,8 @@ extern "C" {
 /* mls_int8_gemm_ws / mls_int4_gemm_ws with a workspace of mlsx_wq_workspace bytes (256-byte
  * aligned; 0: none): shapes whose tiles would not fill the GPU, or whose K is a multiple of
  * 32 but not of 64, run with the reduction axis split over blocks and fp32 partial products
- * in the workspace (gemm_ksplit.hip); every other call is the _ws one. */
+ * in the workspace (gemm_ksplit.hip; at most 384 MiB of them, and of x as three parts, whatever
+ * the rows); every other call is the _ws one. */
 /* The number of ranges that K is split into for such a call, 1: these kernels unsplit, 0: the _ws entry
  * point's kernels (faster there by the models of both). */
 int mlsx_wq_ksplit(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group);

@@ -30,6 +30,7 @@
 // fp32 activations come as PARTS bf16 rows per row of x in 16 PARTS-row groups (row R of the
 // split matrix: part (R / 16) % PARTS of row 16 (R / (16 PARTS)) + R % 16), so that a lane
 // holds all parts of one output in PARTS consecutive accumulator tiles.
+#include <algorithm>
 #include <type_traits>
 
 #include "mfma16.h"
@@ -377,9 +378,14 @@ int launch_shape(const KsArgs& a, int bm, int bn, size_t table, bool partial, hi
   return launch_shape_g<WBITS, MT, OT, PARTS, 0>(a, bm, bn, table, partial, st);
 }
 
+// Most bytes of partial products, and of x as three parts, that a launch works on (the Infinity
+// Cache holds 256 MiB; the largest use at 2048 rows and 11008 columns is 258).
+constexpr int64_t kMostBytes = (int64_t)384 << 20;
+
 struct KsPlan {
   int bm = 0, bn = 0, splits = 0, parts = 1;  // bm 0: not taken
   int unit = 64, units = 0;
+  int64_t rows = 0;  // rows of x a launch; more take several, one after another in one workspace
 };
 
 // k that a range is a multiple of: whole stages and whole groups (32 or multiples of 64)
@@ -391,11 +397,13 @@ int64_t rows_of(const KsPlan& p, int64_t M) { return p.parts == 1 ? M : cdiv(M, 
 int64_t up256(int64_t v) { return cdiv(v, 256) * 256; }
 int64_t ld_part(int64_t N) { return cdiv(N, 4) * 4; }
 int64_t ws_x(const KsPlan& p, int64_t M, int64_t K) { return p.parts == 1 ? 0 : up256(rows_of(p, M) * K * 2); }
+int64_t ws_part(int splits, int64_t M, int64_t N) { return splits > 1 ? splits * M * ld_part(N) * 4 : 0; }
 int64_t ws_need(const KsPlan& p, int64_t M, int64_t N, int64_t K) {
-  return ws_x(p, M, K) + (p.splits > 1 ? (int64_t)p.splits * M * ld_part(N) * 4 : 0);
+  const int64_t m = M < p.rows ? M : p.rows;
+  return ws_x(p, m, K) + ws_part(p.splits, m, N);
 }
 
-int run_plan(int wbits, const KsPlan& pl, const WqArgs& w, uint8_t* ws) {
+int run_rows(int wbits, const KsPlan& pl, const WqArgs& w, uint8_t* ws) {
   KsArgs a{};
   a.a = w.a; a.lda = (int)w.lda;
   a.b = w.w; a.ldb = (int)w.ldw;
@@ -448,6 +456,19 @@ int run_plan(int wbits, const KsPlan& pl, const WqArgs& w, uint8_t* ws) {
   return check_launch("K-split sum");
 }
 
+int run_plan(int wbits, const KsPlan& pl, const WqArgs& w, uint8_t* ws) {
+  const int64_t sz = dt_size(w.a_dt);
+  for (int64_t m = 0; m < w.M; m += pl.rows) {
+    WqArgs c = w;
+    c.a = static_cast<const uint8_t*>(w.a) + m * w.lda * sz;
+    c.c = static_cast<uint8_t*>(w.c) + m * w.ldc * sz;
+    c.M = std::min(pl.rows, w.M - m);
+    const int rc = run_rows(wbits, pl, c, ws);
+    if (rc != MLS_OK) return rc;  // (UNSUPPORTED comes from a tile's limits, so from the first rows)
+  }
+  return MLS_OK;
+}
+
 // What the kernels assume of pointers and strides (the sizes are the plan's).
 bool layout_ok(int wbits, const WqArgs& w) {
   if (!w.a || !w.w || !w.s || !w.c) return false;  // (the general entry points say what is wrong)
@@ -486,13 +507,15 @@ constexpr TileCost kTiles[] = {
     {8, 256, 256, 1, 1.387f, 0.000f, 3.76f, 10.61f, 0.40f, 0.252f},
 };
 
-// The fastest tile and split by the model, its time in us; bm = 0 when nothing fits.
-KsPlan best_tile(int wbits, int64_t M, int64_t N, int64_t K, int group, int parts, float* us) {
+// The fastest tile and split by the model with at most `most` bytes of partial products, its time in
+// us; bm = 0 when nothing fits.
+KsPlan best_tile(int wbits, int64_t M, int64_t N, int64_t K, int group, int parts, int64_t most, float* us) {
   static constexpr int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
   KsPlan best;
   best.parts = parts;
   best.unit = range_unit(wbits, group);
   best.units = (int)cdiv(K, best.unit);
+  best.rows = M;
   *us = 1e30f;
   const int64_t rows = rows_of(best, M);
   const float slow = wbits == 8 || group >= 128 ? 1.0f : group == 64 ? 1.12f : 1.42f;
@@ -506,7 +529,7 @@ KsPlan best_tile(int wbits, int64_t M, int64_t N, int64_t K, int group, int part
     for (int s : kSplits) {
       if (s > best.units) break;
       if (wbits == 4 && cdiv(best.units, s) * (best.unit / group) * t.bn * 4 > 160 * 1024 - 256 * (t.bm + t.bn)) continue;
-      if (s > 1 && any && tiles * s > 800) break;
+      if (s > 1 && ((any && tiles * s > 800) || ws_part(s, M, N) > most)) break;
       any = true;
       const float stages = (float)(cdiv(best.units, s) * (best.unit / 64)) * slow;
       const float r1 = stages * t.t1 + t.edge, r2 = stages * t.t2 + t.edge;
@@ -564,9 +587,31 @@ KsPlan ks_plan(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) 
   const float general = general_us(wbits, M, N, K, a_dt, group, split);
   if (general == 0.0f) return {};
   float us;
-  const KsPlan p = best_tile(wbits, M, N, K, group, !f32 ? 1 : split ? 2 : 3, &us);
+  const int parts = !f32 ? 1 : split ? 2 : 3;
+  KsPlan p = best_tile(wbits, M, N, K, group, parts, INT64_MAX, &us);
+  if (p.bm == 0) return {};
+  auto over = [&](const KsPlan& q) {
+    return ws_part(q.splits, q.rows, N) > kMostBytes || (parts == 3 && ws_x(q, q.rows, K) > kMostBytes);
+  };
+  if (over(p)) {
+    // Past the workspace's bound (groups of 32 at K > 7424: a tile's scale table does not hold all of
+    // K, so K is split however many tiles there are; fp32 x in three parts: 6 bytes a value): other
+    // tiles, or the rows in several launches, whichever the model has faster.
+    p = {};
+    us = 1e30f;
+    for (int64_t rows = M, next = 8192; rows >= 256; rows = next, next /= 2) {
+      if (rows > M) continue;
+      float t;
+      const KsPlan q = best_tile(wbits, rows, N, K, group, parts, kMostBytes, &t);
+      t *= (float)cdiv(M, rows);
+      if (q.bm == 0 || over(q) || t >= us) continue;
+      p = q;
+      us = t;
+    }
+    if (p.bm == 0) return {};
+  }
   if (f32) us += split_estimate_us(M, K);
-  if (p.bm == 0 || us >= general) return {};
+  if (us >= general) return {};
   // whole 192- or 256-column tiles without a split are the engine's own
   if (p.splits == 1 && p.bn > 128 && K % 64 == 0) return {};
   return p;

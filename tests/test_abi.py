@@ -247,3 +247,16 @@ def test_the_k_split_gemm_takes_what_it_is_faster_at(bits, M, N, K, group, taken
     """The plan is compared with the time of the kernel that would otherwise serve the shape, the
     engine's among them (bf16)."""
     assert (kernels.load_library().mlsx_wq_ksplit(bits, M, N, K, kernels.MLS_BF16, group) > 0) == taken
+
+
+@pytest.mark.parametrize("bits,M,N,K,dt,group", [
+    (4, 32768, 4096, 11008, "MLS_BF16", 32), (4, 16384, 11008, 11008, "MLS_F16", 32), (4, 1 << 20, 4096, 8192, "MLS_BF16", 32),
+    (4, 32768, 4096, 11008, "MLS_F32", 32), (4, 32768, 4096, 4128, "MLS_F32", 32), (8, 1 << 20, 1024, 4128, "MLS_F32", 0),
+    (8, 70000, 512, 2080, "MLS_BF16", 0), (4, 300, 1 << 20, 11008, "MLS_BF16", 32), (8, 65536, 4096, 4096, "MLS_F32", 0),
+])
+def test_the_k_split_workspace_is_bounded(bits, M, N, K, dt, group):
+    """Partial products and three-part activations stay within 384 MiB each, at any row count; what the
+    _ws entry point asks for (two parts of fp32 x) comes on top."""
+    L = kernels.load_library()
+    dt = getattr(kernels, dt)
+    assert L.mlsx_wq_workspace(bits, M, N, K, dt, group) <= L.mls_wq_gemm_workspace(bits, M, N, K, dt, group) + (768 << 20)

@@ -130,3 +130,19 @@ def test_short_workspace_takes_the_general_path(dev):
                                       torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     _check(c, x, w, "no workspace")
+
+
+@pytest.mark.parametrize("dtype,bits,M,N,K,group", [
+    (torch.float32, 4, 17000, 72, 4128, 32),     # three parts of x past the bound: rows in two launches
+    (torch.bfloat16, 4, 12289, 4104, 7456, 32),  # a forced split whose partial products pass it
+])
+def test_rows_in_several_launches(dev, dtype, bits, M, N, K, group):
+    """More rows than the workspace's bound allows, the last launch ragged, with strides on both
+    sides; every 97th row and the launches' edges against float64."""
+    q, s, w = _weights(dev, bits, N, K, group, torch.float32, 3)
+    x = torch.randn(M, K + 32, generator=torch.Generator().manual_seed(6)).to(dtype).to(dev)[:, :K]
+    assert kernels.lib().mlsx_wq_workspace(bits, M, N, K, kernels.MLS_F32 if dtype == torch.float32 else kernels.MLS_BF16,
+                                           group) <= 768 << 20
+    y = _run(bits, x, q, s, group)
+    at = torch.tensor(sorted({*range(0, M, 97), 4095, 4096, 8191, 8192, M - 1}), device=dev)
+    _check(y[at], x[at], w, f"{M}x{N}x{K}")
