@@ -622,6 +622,8 @@ int run_ext(int wbits, const WqArgs& w, int c_dt, void* ws, int64_t ws_bytes, bo
   if (c_dt != w.a_dt || !is_float_dt(w.a_dt) || w.M < 1 || w.N < 1 || w.K < 1 || !layout_ok(wbits, w)) return MLS_OK;
   const KsPlan pl = ks_plan(wbits, w.M, w.N, w.K, w.a_dt, w.group);
   if (pl.bm == 0) return MLS_OK;
+  // two parts of fp32 x only where the general path takes two (split_ok); else it multiplies in fp32
+  if (pl.parts == 2 && (!aligned(w.w, 16) || w.ldw % 16 != 0)) return MLS_OK;
   const int64_t need = ws_need(pl, w.M, w.N, w.K);
   if (need && (!ws || ws_bytes < need || !aligned(ws, 256))) return MLS_OK;
   *taken = true;

@@ -146,3 +146,18 @@ def test_rows_in_several_launches(dev, dtype, bits, M, N, K, group):
     y = _run(bits, x, q, s, group)
     at = torch.tensor(sorted({*range(0, M, 97), 4095, 4096, 8191, 8192, M - 1}), device=dev)
     _check(y[at], x[at], w, f"{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("bits,K,group", [(8, 4096, 0), (4, 4096, 64)])
+def test_weights_at_8_of_16_bytes_keep_fp32(dev, bits, K, group):
+    """fp32 x with weights that are 8- but not 16-byte aligned multiplies in fp32, as the general
+    path's split asks for 16. A chain of K fp32 sums rounds by 2^-24 sqrt(K) / 2 of the norm (2e-6
+    here, 1.1e-6 measured); two bf16 parts of x, which keep 2^-16 of it, have 4.9e-6."""
+    M, N = 200, 512
+    q, s, w = _weights(dev, bits, N, K, group, torch.float32, 8)
+    flat = torch.empty(q.numel() + 8, dtype=q.dtype, device=dev)[8:]
+    off = flat.view(q.shape).copy_(q)
+    assert off.data_ptr() % 16 == 8
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(6)).to(dev)
+    want = x.double() @ w.t()
+    assert float((_run(bits, x, off, s, group) - want).norm() / want.norm()) < 2.0 ** -24 * K ** 0.5 / 2
