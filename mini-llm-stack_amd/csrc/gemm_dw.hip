@@ -1,20 +1,20 @@
 // dw[N][K] = dy[M][N]^T x[M][K], all fp32: the master weight's gradient of the INT8
 // straight-through estimator (kernels/autograd_ops.py:132), on the bf16 matrix cores.
 //
-// gfx950 has no fp32 matrix rate near its 16-bit one (4096 x 4096 over 2048 tokens: 496 us in
-// the fp32 library product, 139 TFLOP/s). Here every fp32 value becomes three bf16 parts that
+// gfx950 has no fp32 matrix rate near its 16-bit one (4096 x 4096 over 2048 tokens: 468 us in
+// the fp32 library product, 147 TFLOP/s). Here every fp32 value becomes three bf16 parts that
 // add up to it exactly (8 of its 24 significant bits each, by truncation, so all parts have
 // its sign), and a product becomes the six part products above 2^-24 of it: hi hi, hi mid,
-// mid hi, mid mid, hi lo, lo hi. bf16 keeps fp32's exponent range, so nothing is scaled and
-// small values beside large ones keep their bits.
+// mid hi, mid mid, hi lo, lo hi. bf16 keeps fp32's exponent range, so small values beside large
+// ones keep their bits; and both operands are taken times 2^16, which lifts fp32's smallest value
+// (2^-149) to bf16's (2^-133), so that no bit of any value is lost.
 //
 // Two launches on the caller's stream: dw_parts_kernel transposes both operands into parts with
 // the reduction axis contiguous, [C][3][Mp] (row 3 c + part, Mp = M rounded up to 32, zeros past
 // M), then dw_kernel multiplies. A part read from LDS once feeds two or three products, so the
 // LDS traffic per MFMA is half that of a plain bf16 GEMM and the kernel is bound by the matrix
-// cores: 343 us for both launches at that size, 1.2 PFLOP/s over the six products, the rate of a
-// plain bf16 GEMM. Error against 64 bits there 2.8e-7 of the norm, the library product's 8.1e-7.
-// Parts below bf16's smallest normal (1.2e-38) are lost: values under 1e-33 keep fewer bits.
+// cores: 320 us for both launches at that size, 1.29 PFLOP/s over the six products, the rate
+// of a plain bf16 GEMM. Error against 64 bits there 2.8e-7 of the norm, the library product's 8.1e-7.
 //
 // dw_kernel: block tile BP (rows of dw) x BQ (columns) x 32 tokens, 8 wavefronts of 64 x WTQ
 // outputs, two LDS buffers filled by LDS-direct loads one stage ahead, one barrier a stage.
@@ -23,10 +23,9 @@
 // accumulator of its own and the other five share one, so the large sum is rounded once per 32
 // tokens, not six times.
 //
-// A non-finite value has itself as every part. Where the other operand is finite, a part of it
-// may be zero, and inf * 0 would turn an infinite output into a NaN: a block whose tile comes out
-// with a non-finite value computes it again, with the non-finite parts cleared everywhere but in
-// hi hi, which gives what fp32 arithmetic gives (hi is zero only where the value is).
+// Infinities, NaN, values from 2^112 and sums from 2^96 leave a non-finite value in every tile that
+// they touch: such a block computes its tile again from the operands themselves with fp32 FMAs
+// (whole_tile), which gives what fp32 arithmetic gives, at a fraction of the speed.
 #include <algorithm>
 
 #include "mfma16.h"
@@ -36,6 +35,7 @@ namespace mls {
 namespace {
 
 constexpr int kStage = 32;  // tokens a stage: one MFMA step
+constexpr float kLift = 65536.0f, kDrop = 1.0f / (65536.0f * 65536.0f);  // both operands' 2^16, off again
 
 struct DwParams {
   const uint16_t* p;  // parts of dy [N][3][Mp]
@@ -43,6 +43,10 @@ struct DwParams {
   float* c;
   int64_t ldc;
   int P, Q, Mp;
+  const float* dy;    // the operands themselves (whole_tile)
+  const float* x;
+  int64_t lddy, ldx;
+  int M;
   int p_tiles, q_tiles;
 };
 
@@ -90,7 +94,7 @@ __global__ __launch_bounds__(256) void dw_parts_kernel(const float* __restrict__
       float part[3][2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        const float v = tile[r0 + 2 * h + e][c];
+        const float v = tile[r0 + 2 * h + e][c] * kLift;
         float rest, low;
         split_f32(v, part[0][e], rest);
         split_f32(rest, part[1][e], low);
@@ -138,24 +142,13 @@ __device__ __forceinline__ void stage_sync() {
   asm volatile("" ::: "memory");
 }
 
-// non-finite bf16 values of a pair cleared
-__device__ __forceinline__ uint32_t finite2(uint32_t v) {
-  const uint32_t lo = (v & 0x7F80u) == 0x7F80u ? 0u : v & 0xFFFFu;
-  const uint32_t hi = (v & 0x7F800000u) == 0x7F800000u ? 0u : v & 0xFFFF0000u;
-  return lo | hi;
-}
-__device__ __forceinline__ uint4 finite8(uint4 v) {
-  return make_uint4(finite2(v.x), finite2(v.y), finite2(v.z), finite2(v.w));
-}
-
 template <int BP, int BQ, int WP, int WQ>
 struct DwTile {
   static constexpr int TP = BP / WP / 16, TQ = BQ / WQ / 16;
   static constexpr int P_STAGE = 3 * BP * 64, Q_STAGE = 3 * BQ * 64, STAGE = P_STAGE + Q_STAGE;
   static_assert(WP * WQ == 8, "8 wavefronts");
 
-  // all stages of one tile; CLEAN: non-finite parts only in hi hi
-  template <bool CLEAN>
+  // all stages of one tile
   __device__ static __forceinline__ void run(const DwParams& p, uint8_t* smem, int p0, int q0, int wave, int lane,
                                              f32x4 (&big)[TQ][TP], f32x4 (&rest)[TQ][TP]) {
     const int ld = p.Mp * 2;
@@ -203,22 +196,19 @@ struct DwTile {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < TP; ++j) {
-        const uint4 bh = b[j][0];
-        uint4 bf = bh, bm = b[j][1], bl = b[j][2];
-        if constexpr (CLEAN) bf = finite8(bh), bm = finite8(bm), bl = finite8(bl);
+        const uint4 bh = b[j][0], bm = b[j][1], bl = b[j][2];
         // a product at a time over the tiles: no MFMA waits for the one before it
         using X = Mfma16<__bf16>;
-        auto fin = [](const uint4& v) { return CLEAN ? finite8(v) : v; };
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(fin(a[i][2]), bf, rest[i][j]);
+        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(a[i][2], bh, rest[i][j]);
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(fin(a[i][0]), bl, rest[i][j]);
+        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(a[i][0], bl, rest[i][j]);
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(fin(a[i][1]), bm, rest[i][j]);
+        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(a[i][1], bm, rest[i][j]);
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(fin(a[i][1]), bf, rest[i][j]);
+        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(a[i][1], bh, rest[i][j]);
 #pragma unroll
-        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(fin(a[i][0]), bm, rest[i][j]);
+        for (int i = 0; i < TQ; ++i) rest[i][j] = X::mma(a[i][0], bm, rest[i][j]);
 #pragma unroll
         for (int i = 0; i < TQ; ++i) big[i][j] = X::mma(a[i][0], bh, big[i][j]);
       }
@@ -227,6 +217,52 @@ struct DwTile {
     }
   }
 };
+
+// dw[p0 .. p0 + BP)[q0 .. q0 + BQ) by fp32 FMAs, tokens in order: 16 tokens of both operands in LDS a
+// step, BP / 32 x BQ / 16 outputs a thread.
+template <int BP, int BQ>
+__device__ __forceinline__ void whole_tile(const DwParams& p, float* smem, int p0, int q0) {
+  constexpr int T = 16, RP = BP / 32, RQ = BQ / 16;
+  float (*ds)[BP] = reinterpret_cast<float(*)[BP]>(smem);
+  float (*xs)[BQ] = reinterpret_cast<float(*)[BQ]>(smem + T * BP);
+  const int tid = threadIdx.x, tp = tid / 16, tq = tid % 16;
+  float acc[RP][RQ];
+#pragma unroll
+  for (int i = 0; i < RP; ++i)
+#pragma unroll
+    for (int j = 0; j < RQ; ++j) acc[i][j] = 0.0f;
+  for (int m0 = 0; m0 < p.M; m0 += T) {
+    __syncthreads();
+    const int n = min(T, p.M - m0);
+    for (int t = tid; t < n * BP; t += 512) {
+      const int m = t / BP, c = t % BP;
+      ds[m][c] = p0 + c < p.P ? p.dy[(int64_t)(m0 + m) * p.lddy + p0 + c] : 0.0f;
+    }
+    for (int t = tid; t < n * BQ; t += 512) {
+      const int m = t / BQ, c = t % BQ;
+      xs[m][c] = q0 + c < p.Q ? p.x[(int64_t)(m0 + m) * p.ldx + q0 + c] : 0.0f;
+    }
+    __syncthreads();
+    for (int m = 0; m < n; ++m) {
+      float a[RP], b[RQ];
+#pragma unroll
+      for (int i = 0; i < RP; ++i) a[i] = ds[m][tp + 32 * i];
+#pragma unroll
+      for (int j = 0; j < RQ; ++j) b[j] = xs[m][tq + 16 * j];
+#pragma unroll
+      for (int i = 0; i < RP; ++i)
+#pragma unroll
+        for (int j = 0; j < RQ; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RP; ++i)
+#pragma unroll
+    for (int j = 0; j < RQ; ++j) {
+      const int r = p0 + tp + 32 * i, c = q0 + tq + 16 * j;
+      if (r < p.P && c < p.Q) p.c[(int64_t)r * p.ldc + c] = acc[i][j];
+    }
+}
 
 template <int BP, int BQ, int WP, int WQ>
 __global__ __launch_bounds__(512) void dw_kernel(const DwParams p) {
@@ -238,7 +274,7 @@ __global__ __launch_bounds__(512) void dw_kernel(const DwParams p) {
   const int p0 = pt * BP, q0 = qt * BQ;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   f32x4 big[T::TQ][T::TP], rest[T::TQ][T::TP];
-  T::template run<false>(p, smem, p0, q0, wave, lane, big, rest);
+  T::run(p, smem, p0, q0, wave, lane, big, rest);
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < T::TQ; ++i)
@@ -249,7 +285,10 @@ __global__ __launch_bounds__(512) void dw_kernel(const DwParams p) {
         const float v = big[i][j][r] + rest[i][j][r];
         bad |= (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u;
       }
-  if (__syncthreads_or(bad)) T::template run<true>(p, smem, p0, q0, wave, lane, big, rest);
+  if (__syncthreads_or(bad)) {
+    whole_tile<BP, BQ>(p, reinterpret_cast<float*>(smem), p0, q0);
+    return;
+  }
 
   // lane: dw[p = .. + lane % 16][q = .. + 4 (lane / 16) + r]
   const int lr = lane & 15, g = lane >> 4;
@@ -262,7 +301,7 @@ __global__ __launch_bounds__(512) void dw_kernel(const DwParams p) {
 #pragma unroll
     for (int i = 0; i < T::TQ; ++i) {
       const int col = wq0 + 16 * i + 4 * g;
-      const f32x4 v = big[i][j] + rest[i][j];
+      const f32x4 v = (big[i][j] + rest[i][j]) * kDrop;
       float* dst = p.c + (int64_t)row * p.ldc + col;
       if (v4 && col + 3 < p.Q) {
         *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
@@ -289,8 +328,8 @@ int launch_dw(DwParams p, hipStream_t st) {
 }
 
 // Outputs that the fullest CU computes (one block a CU at a time). The tile with fewer is taken,
-// 256 x 128 where they tie: it reads a quarter less from L2 (4096 x 4096 over 2048 tokens 379 us,
-// 128 x 128 385; 2048 x 2048, 256 tiles of 128 x 128, 140 and 100).
+// 256 x 128 where they tie: it reads a quarter less from L2 (4096 x 4096 over 2048 tokens 320 us,
+// 128 x 128 355; 2048 x 2048, 256 tiles of 128 x 128, 138 and 99).
 int64_t dw_cost(int64_t N, int64_t K, int64_t bp, int64_t bq) {
   return cdiv(cdiv(N, bp) * cdiv(K, bq), 256) * bp * bq;
 }
@@ -311,11 +350,11 @@ extern "C" int64_t mlsx_dw_fp32_workspace(int64_t M, int64_t N, int64_t K) {
   return 6 * Mp * (N + K);
 }
 
-// Against the fp32 library product (us, this and that): 2048 x 4096 x 4096 343 and 496, 256 x 4096 x
-// 4096 67 and 83, 1024 x 2048 x 2048 56 and 64, 1024 x 1024 x 4096 58 and 65, 2048 x 11008 x 4096 971
-// and 1365. Below 2^32 products the launches and the parts weigh too much (256 x 4096 x 2048 38 and
-// 38, 256 x 2048 x 2048 26 and 22), and where the last round of tiles leaves CUs idle the library's
-// smaller tiles win (777 x 2048 x 1024, half of them, 47 and 32).
+// Against the fp32 library product (us, this and that): 2048 x 4096 x 4096 320 and 468, 256 x 4096 x
+// 4096 62 and 73, 1024 x 2048 x 2048 56 and 64, 1024 x 1024 x 4096 58 and 64, 2048 x 11008 x 4096 976
+// and 1368. Below 2^32 products the launches and the parts weigh too much (256 x 4096 x 2048 37 and
+// 36, 256 x 2048 x 2048 25 and 21), and where the last round of tiles leaves CUs idle the library's
+// smaller tiles win (777 x 2048 x 1024, half of them, 47 and 30).
 extern "C" int mlsx_dw_fp32_pays(int64_t M, int64_t N, int64_t K) {
   const int64_t need = mlsx_dw_fp32_workspace(M, N, K);
   if (need == 0 || need > ((int64_t)4 << 30)) return 0;
@@ -344,7 +383,7 @@ extern "C" int mlsx_dw_fp32(const float* dy, int64_t lddy, const float* x, int64
                      dy, lddy, (int)N, x, ldx, (int)K, (int)M, Mp, dyp, xp, vec);
   const int rc = check_launch(fn);
   if (rc != MLS_OK) return rc;
-  const DwParams p{dyp, xp, dw, lddw, (int)N, (int)K, Mp, 0, 0};
+  const DwParams p{dyp, xp, dw, lddw, (int)N, (int)K, Mp, dy, x, lddy, ldx, (int)M, 0, 0};
   if (dw_cost(N, K, 256, 128) <= dw_cost(N, K, 128, 128)) return launch_dw<256, 128, 4, 2>(p, st);
   return launch_dw<128, 128, 2, 4>(p, st);
 }

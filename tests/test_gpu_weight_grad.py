@@ -69,6 +69,32 @@ def test_non_finite_as_fp32():
 
 
 @gpu
+@pytest.mark.parametrize("sd,sx", [(1e-36, 1.0), (1e4, 1e-38), (1e-20, 1e-16), (1e34, 1e-36), (3e33, 1e2), (1e16, 1e17), (1e-41, 1e20)])
+def test_every_scale_keeps_its_bits(sd, sx):
+    """Values near fp32's smallest, whole or beside ordinary columns, and values and sums so large that
+    the parts pass bf16's range, are as close to float64 as fp32 sums are."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    dy = torch.randn(96, 300, generator=g, device="cuda")
+    x = torch.randn(96, 200, generator=g, device="cuda")
+    for cols in (slice(None), slice(7, 9)):
+        a, b = dy.clone(), x.clone()
+        a[:, cols] *= sd
+        b[:, cols] *= sx
+        err = (_dw(a, b).double() - a.double().t() @ b.double()).abs()
+        assert (err <= _bound(a, b) + 96 * 2.0**-149).all()
+
+
+@gpu
+def test_infinity_times_the_smallest_values():
+    """An infinity times a value whose parts are small stays an infinity of its sign, as in fp32."""
+    dy = torch.logspace(-44.5, 5, 257, device="cuda").repeat(40, 1) * torch.where(torch.arange(257, device="cuda") % 2 == 0, 1.0, -1.0)
+    x = torch.ones(40, 130, device="cuda")
+    x[11, 3] = float("-inf")
+    got = _dw(dy, x)[:, 3]
+    assert torch.equal(got, dy[11] * x[11, 3]) and torch.isinf(got).all()
+
+
+@gpu
 def test_route():
     """Where the kernel serves the gradient, and where torch must: a gradient of the gradient,
     16-bit and few tokens."""
