@@ -3,7 +3,7 @@
 // blocks, the fp32 partial products summed by a second kernel.
 //
 // The dense engine (gemm_mfma16.hip) gives every block all of K. A prompt chunk of 333 rows
-// through a 11008 -> 4096 projection is then 32 blocks of 256 x 128 (or 176 of 32 x 256, a
+// through a 11008 -> 4096 projection is then 64 blocks of 256 x 128 (or 176 of 32 x 256, a
 // wavefront a SIMD) that each walk 172 stages of 64 k. Here the same tiles are cut into S
 // ranges of K, so that about two rounds of 256 blocks share the walk.
 //
@@ -578,7 +578,7 @@ float general_us(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group
 //
 // fp32 activations: two bf16 parts where the general path takes two (K % 64 == 0, INT4 groups
 // a multiple of 64, M >= 2), and three, which hold x exactly, where it multiplies in fp32
-// (error against 64 bits at 200 x 4096 x 4096, groups of 32: 3.6e-7 in fp32, 3.0e-7 here).
+// (error against 64 bits at 200 x 4096 x 4096, groups of 32: 3.6e-7 in fp32, 1.5e-7 here).
 KsPlan ks_plan(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) {
   if (K % 32 != 0 || K < 64 || M > (1 << 24) || N > (1 << 28) || K * 512 >= (1ll << 31)) return {};
   if (wbits == 4 && ((group != 32 && group % 64 != 0) || group < 32 || group > (1 << 20) || K % group != 0)) return {};

@@ -42,8 +42,8 @@ def int8_matmul(a: torch.Tensor, w_q: torch.Tensor, scale: torch.Tensor):
     s, sdt = scale_vector(scale.reshape(-1).contiguous())
     c = torch.empty(M, N, dtype=a.dtype, device=dev)
     lib = kernels.lib()
-    # fp32 activations with M >= 2 run on the matrix cores as bf16 hi + lo parts, split
-    # into a workspace from torch's caching allocator; other calls need none
+    # workspace from torch's caching allocator: fp32 activations with M >= 2 as bf16 parts for the
+    # matrix cores, and the fp32 partial products of calls whose K is split over blocks
     need = lib.mlsx_wq_workspace(8, M, N, K, adt, 0)
     ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
     kernels.check(lib.mlsx_int8_gemm(
