@@ -52,8 +52,8 @@ def _check(y, x, w, what, split=False):
 ])
 def test_shapes(dev, bits, M, N, K, group, dtype):
     """Ragged rows, columns and K (a multiple of 32) with NaN beside the operand's rows: whatever
-    a tile reads past K or M must not reach a result. (The sizes are ones the K-split kernels
-    take: more rows than the skinny and medium kernels serve faster.)"""
+    a tile reads past K or M must not reach a result. (All but the smallest two INT4 sizes are
+    ones the K-split kernels take: more rows than the skinny and medium kernels serve faster.)"""
     q, s, w = _weights(dev, bits, N, K, group, torch.float32 if M % 2 else torch.float16, K + M)
     pad = torch.full((M + 1, K + 32), float("nan"), device=dev, dtype=dtype)
     x = pad[:M, :K]
@@ -153,7 +153,8 @@ def test_weights_at_8_of_16_bytes_keep_fp32(dev, bits, K, group):
     """fp32 x with weights that are 8- but not 16-byte aligned multiplies in fp32, as the general
     path's split asks for 16. A chain of K fp32 sums rounds by 2^-24 sqrt(K) / 2 of the norm (2e-6
     here, 1.1e-6 measured); two bf16 parts of x, which keep 2^-16 of it, have 4.9e-6."""
-    M, N = 200, 512
+    M, N = 333, 1024
+    assert kernels.lib().mlsx_wq_ksplit(bits, M, N, K, kernels.MLS_F32, group) > 0  # (aligned, it is split)
     q, s, w = _weights(dev, bits, N, K, group, torch.float32, 8)
     flat = torch.empty(q.numel() + 8, dtype=q.dtype, device=dev)[8:]
     off = flat.view(q.shape).copy_(q)
