@@ -548,18 +548,21 @@ KsPlan best_tile(int wbits, int64_t M, int64_t N, int64_t K, int group, int part
 }
 
 // What the general entry points would take for a shape, in us (0: always theirs; infinity: the kernel
-// with one thread an output).
-float general_us(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group, bool split) {
+// with one thread an output). *fitted: by the engine's model, which was fitted together with the
+// K-split kernels' times (and with the pass that splits fp32 x); the others are off by a tenth or so.
+float general_us(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group, bool split, bool* fitted) {
+  *fitted = true;
   const bool f32 = a_dt == MLS_F32;
   const int ks = wbits == 4 && group % 128 == 0 ? 128 : 64;  // k a step of the skinny and medium kernels
   const bool stepped = K % ks == 0 && (wbits == 8 || group % 64 == 0);
   if (M > 16 && (f32 ? split : stepped)) {
     const int64_t m = split ? split_rows(M) : M, bm = split && wbits == 8 && m >= 256 ? 256 : 128;
     if ((split ? m <= 512 : M <= 256) && cdiv(m, bm) * cdiv(N, 256) < 128)
-      return small_estimate_us(wbits, m, N, K, group, f32 ? 4 : 2, split);
+      return *fitted = false, small_estimate_us(wbits, m, N, K, group, f32 ? 4 : 2, split);
     return engine_estimate_us(wbits, m, N, K, group, split);
   }
   if (M > 16 && !f32 && K % 64 == 0) return engine_estimate_us(wbits, M, N, K, group, false);
+  *fitted = false;
   if (M > 1 && M <= 16 && stepped) return 0.0f;     // the skinny MFMA kernel
   // the register GEMVs: a pass over the weights for every `rows` rows of x (their registers
   // hold rows * K / 64 values a lane); measured 0.2 us a pass plus 0.15
@@ -584,7 +587,8 @@ KsPlan ks_plan(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) 
   if (wbits == 4 && ((group != 32 && group % 64 != 0) || group < 32 || group > (1 << 20) || K % group != 0)) return {};
   const bool f32 = a_dt == MLS_F32;
   const bool split = f32 && M > 1 && K % 64 == 0 && (wbits == 8 || group % 64 == 0);
-  const float general = general_us(wbits, M, N, K, a_dt, group, split);
+  bool fitted;
+  const float general = general_us(wbits, M, N, K, a_dt, group, split, &fitted);
   if (general == 0.0f) return {};
   float us;
   const int parts = !f32 ? 1 : split ? 2 : 3;
@@ -610,8 +614,7 @@ KsPlan ks_plan(int wbits, int64_t M, int64_t N, int64_t K, int a_dt, int group) 
     }
     if (p.bm == 0) return {};
   }
-  if (f32) us += split_estimate_us(M, K);
-  if (us >= general) return {};
+  if (fitted ? us + (f32 ? split_estimate_us(M, K) : 0.0f) >= general : us >= 0.92f * general) return {};
   // whole 192- or 256-column tiles without a split are the engine's own
   if (p.splits == 1 && p.bn > 128 && K % 64 == 0) return {};
   return p;
