@@ -285,7 +285,9 @@ __global__ __launch_bounds__(64 * WM * WN) void ksplit_kernel(const KsArgs p) {
       for (int r = 0; r < 4; ++r) {
         float t = acc[i][jo * PARTS + PARTS - 1][r];  // the smallest part first
 #pragma unroll
-        for (int part = PARTS - 2; part >= 0; --part) t += acc[i][jo * PARTS + part][r];
+        for (int part = PARTS - 2; part >= 0; --part)
+          t = PARTS == 3 ? fmaf(t, 1.0f / 256.0f, acc[i][jo * PARTS + part][r])  // (part p is stored times 2^8p)
+                         : t + acc[i][jo * PARTS + part][r];
         v[r] = t * sn[r];
       }
       OT* dst = c + (int64_t)m * p.ldc + nb;

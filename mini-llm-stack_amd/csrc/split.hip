@@ -54,8 +54,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
 
 // Three parts: hi = x truncated to bf16, mid = x - hi truncated to bf16, lo = the rest. Each
 // takes 8 of the 24 significant bits (the differences are exact in fp32), so the three add up
-// to x exactly. Non-finite x: hi = x, the others 0. Row m's part t is row 48 (m / 16) +
-// 16 t + m % 16.
+// to x exactly. mid is stored times 2^8 and lo times 2^16 (neither passes 2 |x|, so neither
+// overflows): the bits of the smallest values, down to 2^-149, would lie below bf16's 2^-133.
+// Non-finite x: hi = x, the others 0. Row m's part t is row 48 (m / 16) + 16 t + m % 16.
 template <bool VEC>
 __global__ __launch_bounds__(256) void split_rows3_kernel(const float* __restrict__ x, int64_t ldx, int M, int K,
                                                           __bf16* __restrict__ x2, int Mp) {
@@ -84,8 +85,10 @@ __global__ __launch_bounds__(256) void split_rows3_kernel(const float* __restric
     float h0, h1, r0, r1, d0, d1, l0, l1;
     split_f32(v[2 * q], h0, r0);
     split_f32(v[2 * q + 1], h1, r1);
-    split_f32(r0, d0, l0);
-    split_f32(r1, d1, l1);
+    split_f32(r0 * 256.0f, d0, l0);
+    split_f32(r1 * 256.0f, d1, l1);
+    l0 *= 256.0f;
+    l1 *= 256.0f;
     h[q] = pack2_bits((__bf16)h0, (__bf16)h1);  // (all exact)
     d[q] = pack2_bits((__bf16)d0, (__bf16)d1);
     l[q] = pack2_bits((__bf16)l0, (__bf16)l1);

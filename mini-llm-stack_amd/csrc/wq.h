@@ -67,7 +67,7 @@ int launch_split_rows(const float* x, int64_t ldx, int64_t M, int64_t K, void* x
 inline float split_estimate_us(int64_t M, int64_t K) { return 1.7f + 2.0e-6f * (float)M * (float)K; }
 // x fp32 [M][ldx] -> `parts` (2 or 3) bf16 rows per row, row m's part t at row
 // 16 parts (m / 16) + 16 t + m % 16 of x2 [16 parts ceil(M / 16)][K] (zeros past M): hi + lo
-// (x to 2^-16), or three parts that add up to x exactly.
+// (x to 2^-16), or three parts, part t times 2^8t, that add up to x exactly.
 int launch_split_parts(const float* x, int64_t ldx, int64_t M, int64_t K, int parts, void* x2, hipStream_t st);
 // The GEMM of split rows q.a ([q.M][q.lda] bf16, q.M = split_rows(m_out)) into fp32 q.c:
 // the medium GEMM where the engine would have few tiles, else the engine.

@@ -162,3 +162,16 @@ def test_weights_at_8_of_16_bytes_keep_fp32(dev, bits, K, group):
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(6)).to(dev)
     want = x.double() @ w.t()
     assert float((_run(bits, x, off, s, group) - want).norm() / want.norm()) < 2.0 ** -24 * K ** 0.5 / 2
+
+
+@pytest.mark.parametrize("scale", [1e-36, 1e-40, 1.0, 1e34])
+@pytest.mark.parametrize("bits,M,N,K,group", [(4, 200, 264, 2048, 32), (8, 300, 264, 2080, 0)])
+def test_three_parts_hold_every_value(dev, bits, M, N, K, group, scale):
+    """fp32 x in three bf16 parts is x itself at every magnitude, so the outputs are as close to float64
+    as fp32 sums are (the smallest: to the last place of a subnormal output)."""
+    assert kernels.lib().mlsx_wq_ksplit(bits, M, N, K, kernels.MLS_F32, group) > 0
+    q, s, w = _weights(dev, bits, N, K, group, torch.float32, 12)
+    x = (torch.randn(M, K, generator=torch.Generator().manual_seed(6)) * scale).to(dev)
+    y, want = _run(bits, x, q, s, group).double(), x.double() @ w.t()
+    terms = (x.double().square() @ w.square().t()).sqrt()
+    assert float(((y - want).abs() - 2.0 ** -17 * terms - 2.0 ** -148).max()) <= 0
